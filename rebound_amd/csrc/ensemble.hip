@@ -92,6 +92,7 @@ static WHParams ens_params(const Ensemble* e) {
     P.G = e->G;
     P.soft2 = 0.;
     P.compensated = e->compensated;
+    P.all_active = 1;
     P.nsteps = 0;
     P.safe_mode = e->safe_mode;
     P.did_modify = 0;

@@ -337,6 +337,7 @@ static WHParams pool_params(Server* S, int ntasks, long nsteps) {
     W.stride = P.cap;
     W.G = 1.;   // per system: WHSys::G
     W.soft2 = 0.;
+    W.all_active = 1;
     W.compensated = 0;
     W.nsteps = nsteps;
     W.safe_mode = 0;

@@ -56,6 +56,7 @@ struct WHParams {
     int corrector = 0;        // first symplectic corrector order (Jacobi): 0, 3, 5, 7, 11, 17
     int corrector2 = 0;       // second corrector (Jacobi): 0 or 1
     int kernel = 0;           // 0 default, 1 modified kick, 2 composition, 3 lazy (Jacobi)
+    int all_active = 0;       // no test particles: every system has Nact == Nact_grav == N
     int jacgrav = 0;          // accelerations by the Jacobi gravity (kernels 1 and 3)
     // First-order variational equations (Jacobi).  `pv` holds the inertial
     // variational particles (fields x y z vx vy vz ax ay az m, `vstride`
@@ -78,6 +79,10 @@ struct WHParams {
 constexpr int kMegnoFields = 9;
 
 int whfast_launch(const WHParams& P, hipStream_t st);
+// The one-lane-per-planet kernels for all-active systems (whfast_lane.hip).
+bool whfast_lane_takes(const WHParams& P);
+void whfast_lane_launch(const WHParams& P, hipStream_t st);
+int whfast_lane_per_cu();
 int whfast_energy_launch(const WHParams& P, double* out, int nsys, hipStream_t st);
 int whfast_group_size(int K);
 int whfast_max_resident(int device);
