@@ -62,8 +62,9 @@ REB_API int reb_amd_kernel_time(struct reb_simulation* r, double* total_ms, int*
 /* With profiling on: the ordered body pairs the timed direct-gravity kernels
  * evaluated since profiling was switched on or last read (then reset).  On
  * the symmetric path (every body active, no ghost boxes, nothing ignored,
- * N >= 8192) the timed kernel covers the pairs between superblocks of 1024
- * bodies, N^2 minus the pairs inside superblocks; otherwise N(N-1). */
+ * N >= 8192) the pairs between superblocks of 1024 bodies, N^2 minus the pairs
+ * inside superblocks (which the same launch evaluates, not counted);
+ * otherwise N(N-1). */
 REB_API double reb_amd_kernel_pairs(struct reb_simulation* r);
 
 /* ------------------------------------------------------------ device forces

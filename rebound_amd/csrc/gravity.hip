@@ -690,10 +690,10 @@ __global__ __launch_bounds__(256) void k_seg_reduce(const SegJob* __restrict__ j
 // fused multiply-adds on each side; per step the rotation adds six moves.
 //
 // Outputs, all in fixed order (the results are deterministic):
-//   ipart[t][c][SB]  target-side sums of task t (targets of A, sources of B)
+//   ipart[t][p][c][SB]  target-side sums of part p of task t (targets of A, sources of B)
 //   jpart[t][c][SB]  source-side sums of task t (bodies of B, all targets of A)
 //                    with the sign of the term for A's bodies: S_j = -jpart
-//   dpart[6][N]      the one-sided sums within each superblock (direct_fast_block)
+//   dpart[d][6][N]   the one-sided sums within each superblock, 256 sources each (direct_fast_block)
 // and k_sym_reduce adds, per body, the partials of every superblock in
 // ascending order with Kahan compensation.
 #ifndef RB_SYM_TPL
@@ -703,6 +703,7 @@ static constexpr int kSymTPL = RB_SYM_TPL;           // targets per lane
 static constexpr int kSymSB = 4 * 64 * kSymTPL;       // bodies per superblock
 static constexpr int kSymJB = 64;                     // sources per J-block
 static constexpr int kSymMinN = 8192;                 // below: the one-sided kernel
+static constexpr int kSymDiag = kSymSB / kFast;       // source tiles of a superblock (one-sided pairs)
 
 // Lane k receives lane k-1's value, lane 0 lane 63's (DPP wave_ror:1).
 __device__ __forceinline__ double dpp_ror1(double v) {
@@ -715,107 +716,132 @@ __host__ __device__ __forceinline__ int sym_task(int A, int B, int nsb) {
     return A * nsb - A * (A + 1) / 2 + (B - A - 1);
 }
 
+// One J-block's 64 steps for the lane's targets.  CHECK: the J-block is the
+// last, ragged one of the bodies (its first jlim sources exist).
 template <int MODE, bool CHECK>
+__device__ __forceinline__ void sym_jblock(const double4* __restrict__ src, int k, int jlim, const double* tx,
+                                           const double* ty, const double* tz, const double* tm, double soft2,
+                                           double c15, double c1875, double* bx, double* by, double* bz, double& jx,
+                                           double& jy, double& jz) {
+#pragma unroll 4
+    for (int s = 0; s < kSymJB; s++) {
+        const int idx = (k - s) & (kSymJB - 1);     // the source's index in the J-block
+        const double4 sj = src[k + kSymJB - s];
+#pragma unroll
+        for (int q = 0; q < kSymTPL; q++) {
+            const double dx = tx[q] - sj.x;
+            const double dy = ty[q] - sj.y;
+            const double dz = tz[q] - sj.z;
+            const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, soft2)));
+            double wr;
+            if (MODE == FM_SPLIT) {
+                const double yv = (double)__builtin_amdgcn_rsqf((float)r2);
+                wr = yv * yv * yv;
+            } else {
+                wr = rinv3_fp64(r2, c15, c1875);
+            }
+            if (CHECK && idx >= jlim) wr = 0.;
+            const double wj = wr * sj.w;
+            const double wi = wr * tm[q];
+            bx[q] = fma(wj, dx, bx[q]);
+            by[q] = fma(wj, dy, by[q]);
+            bz[q] = fma(wj, dz, bz[q]);
+            jx = fma(wi, dx, jx);
+            jy = fma(wi, dy, jy);
+            jz = fma(wi, dz, jz);
+        }
+        jx = dpp_ror1(jx);
+        jy = dpp_ror1(jy);
+        jz = dpp_ror1(jz);
+    }
+}
+
+// Workgroups [0, ntasks * split): part p of task (A, B) takes 1/split of B's
+// J-blocks.  One workgroup per task leaves most of the chip idle below ~40000
+// bodies (8192 bodies are 28 tasks for 256 CUs), so sym_split cuts the tasks.
+// The remaining workgroups evaluate the pairs inside the superblocks
+// (one-sided, 256 targets x 256 sources each); they are short and fill the
+// launch's tail.  One launch for full and ragged tasks alike (10007 bodies took
+// 237 + 221 us in two).
+template <int MODE>
 __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, const double* __restrict__ m,
-                                                    int N, int nsb, double soft2, const int2* __restrict__ tasks,
-                                                    int ntasks_done, double* __restrict__ ipart,
-                                                    double* __restrict__ jpart) {
+                                                    int N, int nsb, int ntasks, int split, double soft2,
+                                                    const int2* __restrict__ tasks, double* __restrict__ ipart,
+                                                    double* __restrict__ jpart, double* __restrict__ dpart) {
     // J-block sources (x, y, z, m), double-buffered, each stored twice in a
     // row so that lane k reads entry k + 64 - s at step s without wrapping
     __shared__ double4 jt[2][2 * kSymJB];
     __shared__ double jred[2][4][3][kSymJB];       // per-wave source sums of a J-block
-    const int2 tk = tasks[ntasks_done + blockIdx.x];
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= ntasks * split) {
+        static_assert(sizeof(jt) >= sizeof(double4) * kFast, "the one-sided tile fits the J-block buffers");
+        const int u = (int)blockIdx.x - ntasks * split;
+        const int bx = u / kSymDiag;
+        const int j0 = bx * kFast / kSymSB * kSymSB;
+        direct_fast_block<MODE>(x, y, z, m, N, j0, min(N, j0 + kSymSB), kFast, 0, soft2, GBZero{}, dpart, N, bx,
+                                u % kSymDiag, &jt[0][0]);
+        return;
+    }
+    const int2 tk = tasks[blockIdx.x % ntasks];
+    const int part = (int)blockIdx.x / ntasks;
     const int A = tk.x, B = tk.y;
     const int t = sym_task(A, B, nsb);
-    const int tid = threadIdx.x;
     const int w = tid >> 6, k = tid & 63;
-    // targets of this lane
+    // targets of this lane (A < B: never the ragged superblock)
     double tx[kSymTPL], ty[kSymTPL], tz[kSymTPL], tm[kSymTPL];
     double sx[kSymTPL], sy[kSymTPL], sz[kSymTPL];
 #pragma unroll
     for (int q = 0; q < kSymTPL; q++) {
         const int i = A * kSymSB + w * 64 * kSymTPL + q * 64 + k;
-        const bool ok = !CHECK || i < N;
-        tx[q] = ok ? x[i] : 0.;
-        ty[q] = ok ? y[i] : 0.;
-        tz[q] = ok ? z[i] : 0.;
-        tm[q] = ok ? m[i] : 0.;
+        tx[q] = x[i];
+        ty[q] = y[i];
+        tz[q] = z[i];
+        tm[q] = m[i];
         sx[q] = sy[q] = sz[q] = 0.;
     }
     const int jbase = B * kSymSB;
     constexpr int NJB = kSymSB / kSymJB;
-    // prologue: J-block 0 into LDS, J-block 1 into registers
+    const int jb0 = part * NJB / split;
+    const int jb1 = min((part + 1) * NJB / split, (N - jbase + kSymJB - 1) / kSymJB);
+    auto source = [&](int jb) {
+        const int j = jbase + jb * kSymJB + tid;
+        return jb < jb1 && j < N ? make_double4(x[j], y[j], z[j], m[j]) : make_double4(0., 0., 0., 0.);
+    };
+    // prologue: the first J-block into LDS, the second into registers
     double4 nxt = make_double4(0., 0., 0., 0.);
     if (tid < kSymJB) {
-        const int j0 = jbase + tid;
-        const bool ok0 = !CHECK || j0 < N;
-        const double4 v0 = ok0 ? make_double4(x[j0], y[j0], z[j0], m[j0]) : make_double4(0., 0., 0., 0.);
-        jt[0][tid] = v0;
-        jt[0][tid + kSymJB] = v0;
-        const int j1 = jbase + kSymJB + tid;
-        const bool ok1 = !CHECK || j1 < N;
-        if (ok1) nxt = make_double4(x[j1], y[j1], z[j1], m[j1]);
+        const double4 v0 = source(jb0);
+        jt[jb0 & 1][tid] = v0;
+        jt[jb0 & 1][tid + kSymJB] = v0;
+        nxt = source(jb0 + 1);
     }
+    // source sums of a finished J-block: the four waves' in order
+    auto flush = [&](int jb) {
+        if (w >= 3) return;
+        const double* r = &jred[jb & 1][0][w][k];
+        const double v = ((r[0] + r[3 * kSymJB]) + r[6 * kSymJB]) + r[9 * kSymJB];
+        jpart[((size_t)t * 3 + w) * kSymSB + jb * kSymJB + k] = v;
+    };
     const double c15 = vreg_const(1.5);
     const double c1875 = vreg_const(1.875);
-    for (int jb = 0; jb < NJB; jb++) {
+    for (int jb = jb0; jb < jb1; jb++) {
         __syncthreads();
-        if (jb > 0 && w < 3) {
-            // source sums of J-block jb-1: the four waves' in order
-            const double* r = &jred[(jb - 1) & 1][0][w][k];
-            const double v = ((r[0] + r[3 * kSymJB]) + r[6 * kSymJB]) + r[9 * kSymJB];
-            jpart[((size_t)t * 3 + w) * kSymSB + (jb - 1) * kSymJB + k] = v;
-        }
+        if (jb > jb0) flush(jb - 1);
         if (tid < kSymJB) {
-            if (jb + 1 < NJB) {
-                jt[(jb + 1) & 1][tid] = nxt;
-                jt[(jb + 1) & 1][tid + kSymJB] = nxt;
-            }
-            const int jn = jbase + (jb + 2) * kSymJB + tid;
-            const bool okn = jb + 2 < NJB && (!CHECK || jn < N);
-            nxt = okn ? make_double4(x[jn], y[jn], z[jn], m[jn]) : make_double4(0., 0., 0., 0.);
+            jt[(jb + 1) & 1][tid] = nxt;
+            jt[(jb + 1) & 1][tid + kSymJB] = nxt;
+            nxt = source(jb + 2);
         }
-        const double4* src = jt[jb & 1];
         double bx[kSymTPL], by[kSymTPL], bz[kSymTPL];
 #pragma unroll
         for (int q = 0; q < kSymTPL; q++) bx[q] = by[q] = bz[q] = 0.;
         double jx = 0., jy = 0., jz = 0.;
-        const int jlim = CHECK ? N - (jbase + jb * kSymJB) : kSymJB;   // valid sources of this J-block
-#pragma unroll 4
-        for (int s = 0; s < kSymJB; s++) {
-            const int idx = (k - s) & (kSymJB - 1);     // the source's index in the J-block
-            const double4 sj = src[k + kSymJB - s];
-#pragma unroll
-            for (int q = 0; q < kSymTPL; q++) {
-                const double dx = tx[q] - sj.x;
-                const double dy = ty[q] - sj.y;
-                const double dz = tz[q] - sj.z;
-                const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, soft2)));
-                double wr;
-                if (MODE == FM_SPLIT) {
-                    const double yv = (double)__builtin_amdgcn_rsqf((float)r2);
-                    wr = yv * yv * yv;
-                } else {
-                    wr = rinv3_fp64(r2, c15, c1875);
-                }
-                if (CHECK) {
-                    const int i = A * kSymSB + w * 64 * kSymTPL + q * 64 + k;
-                    if (i >= N || idx >= jlim) wr = 0.;
-                }
-                const double wj = wr * sj.w;
-                const double wi = wr * tm[q];
-                bx[q] = fma(wj, dx, bx[q]);
-                by[q] = fma(wj, dy, by[q]);
-                bz[q] = fma(wj, dz, bz[q]);
-                jx = fma(wi, dx, jx);
-                jy = fma(wi, dy, jy);
-                jz = fma(wi, dz, jz);
-            }
-            jx = dpp_ror1(jx);
-            jy = dpp_ror1(jy);
-            jz = dpp_ror1(jz);
-        }
+        const int jlim = N - (jbase + jb * kSymJB);
+        if (jlim >= kSymJB)
+            sym_jblock<MODE, false>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, bx, by, bz, jx, jy, jz);
+        else
+            sym_jblock<MODE, true>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, bx, by, bz, jx, jy, jz);
 #pragma unroll
         for (int q = 0; q < kSymTPL; q++) {
             sx[q] += bx[q];
@@ -828,61 +854,88 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
         jr[2 * kSymJB] = jz;
     }
     __syncthreads();
-    if (w < 3) {
-        const double* r = &jred[(NJB - 1) & 1][0][w][k];
-        const double v = ((r[0] + r[3 * kSymJB]) + r[6 * kSymJB]) + r[9 * kSymJB];
-        jpart[((size_t)t * 3 + w) * kSymSB + (NJB - 1) * kSymJB + k] = v;
-    }
+    if (jb1 > jb0) flush(jb1 - 1);
 #pragma unroll
     for (int q = 0; q < kSymTPL; q++) {
         const int li = w * 64 * kSymTPL + q * 64 + k;
-        double* p = ipart + (size_t)t * 3 * kSymSB + li;
+        double* p = ipart + ((size_t)t * split + part) * 3 * kSymSB + li;
         p[0] = sx[q];
         p[kSymSB] = sy[q];
         p[2 * kSymSB] = sz[q];
     }
 }
 
-// The one-sided sums inside each superblock (pairs i != j of one superblock):
-// the fast pair block with targets and sources limited to the superblock.
-template <int MODE>
-__global__ __launch_bounds__(kFast) __attribute__((amdgpu_waves_per_eu(RB_FAST_WAVES, RB_FAST_WAVES))) void k_direct_diag(
-    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
-    const double* __restrict__ m, int N, double soft2, double* __restrict__ dpart) {
-    __shared__ double4 tile[kFast];
-    constexpr int per = kSymSB / kFast;                 // target blocks per superblock
-    const int A = (int)blockIdx.x / per;
-    const int j0 = A * kSymSB;
-    const int j1 = min(N, j0 + kSymSB);
-    direct_fast_block<MODE>(x, y, z, m, N, j0, j1, kSymSB, 0, soft2, GBZero{}, dpart, N, (int)blockIdx.x, 0, tile);
-}
-
 // Per body: the partials of every superblock in ascending order (Kahan), then
-// -G and the fused kick and drift as in the one-sided reduction.
-__global__ void k_sym_reduce(const double* __restrict__ ipart, const double* __restrict__ jpart,
-                             const double* __restrict__ dpart, int N, int nsb, double negG, double* __restrict__ ax,
-                             double* __restrict__ ay, double* __restrict__ az, KickDrift kd) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int X = i / kSymSB, loc = i % kSymSB;
+// -G and the fused kick and drift as in the one-sided reduction.  A workgroup
+// takes 64 bodies of one superblock; its four wavefronts each sum a quarter of
+// the partials (the loads of eight in flight), and the first adds the four
+// sums in order.  A body of superblock X has X source-side sums, kSymDiag one-sided
+// sums with their carries, and `split` target-side sums per later superblock.
+__global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ ipart,
+                                                    const double* __restrict__ jpart,
+                                                    const double* __restrict__ dpart, int N, int nsb, int split,
+                                                    double negG, double* __restrict__ ax, double* __restrict__ ay,
+                                                    double* __restrict__ az, KickDrift kd) {
+    __shared__ double sums[4][6][64];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int first = (int)blockIdx.x * 64;
+    const int i = first + lane;
+    const int X = first / kSymSB, loc = first % kSymSB;
+    const int ii = min(i, N - 1) - first;          // lanes past the end read the last body's
     double s[3] = {0., 0., 0.}, c[3] = {0., 0., 0.};
-    for (int Y = 0; Y < nsb; Y++) {
-        if (Y < X) {
-            const double* p = jpart + (size_t)sym_task(Y, X, nsb) * 3 * kSymSB + loc;
-#pragma unroll
-            for (int q = 0; q < 3; q++) kahan_add(-p[(size_t)q * kSymSB], s[q], c[q]);
-        } else if (Y == X) {
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                kahan_add(dpart[(size_t)q * N + i], s[q], c[q]);
-                kahan_add(-dpart[(size_t)(q + 3) * N + i], s[q], c[q]);
-            }
+    const int total = X + 2 * kSymDiag + (nsb - 1 - X) * split;
+    const int e0 = total * w / 4, e1 = total * (w + 1) / 4;
+    // entry e: base pointer of its first component, component stride, sign
+    auto load = [&](int e, double* v) {
+        const double* p;
+        size_t stride = kSymSB;
+        double sign = 1.;
+        if (e < X) {
+            p = jpart + (size_t)sym_task(e, X, nsb) * 3 * kSymSB + loc;
+            sign = -1.;
+        } else if (e < X + 2 * kSymDiag) {
+            const int q = e - X;
+            p = dpart + ((size_t)(q >> 1) * 6 + (q & 1 ? 3 : 0)) * N + first;
+            stride = N;
+            sign = q & 1 ? -1. : 1.;
         } else {
-            const double* p = ipart + (size_t)sym_task(X, Y, nsb) * 3 * kSymSB + loc;
-#pragma unroll
-            for (int q = 0; q < 3; q++) kahan_add(p[(size_t)q * kSymSB], s[q], c[q]);
+            const int q = e - X - 2 * kSymDiag;
+            p = ipart + ((size_t)sym_task(X, X + 1 + q / split, nsb) * split + q % split) * 3 * kSymSB + loc;
         }
+#pragma unroll
+        for (int f = 0; f < 3; f++) v[f] = sign * p[f * stride + ii];
+    };
+    constexpr int BATCH = 8;
+    int e = e0;
+    for (; e + BATCH <= e1; e += BATCH) {
+        double v[BATCH][3];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) load(e + u, v[u]);
+#pragma unroll
+        for (int u = 0; u < BATCH; u++)
+#pragma unroll
+            for (int f = 0; f < 3; f++) kahan_add(v[u][f], s[f], c[f]);
     }
+    for (; e < e1; e++) {
+        double v[3];
+        load(e, v);
+#pragma unroll
+        for (int f = 0; f < 3; f++) kahan_add(v[f], s[f], c[f]);
+    }
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        sums[w][f][lane] = s[f];
+        sums[w][f + 3][lane] = c[f];
+    }
+    __syncthreads();
+    if (w != 0 || i >= N) return;
+#pragma unroll
+    for (int g = 1; g < 4; g++)
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            kahan_add(sums[g][f][lane], s[f], c[f]);
+            kahan_add(-sums[g][f + 3][lane], s[f], c[f]);
+        }
     const double o0 = negG * s[0], o1 = negG * s[1], o2 = negG * s[2];
     ax[i] = o0;
     ay[i] = o1;
@@ -904,36 +957,52 @@ __global__ void k_sym_reduce(const double* __restrict__ ipart, const double* __r
 struct SymPlan {
     int nsb = 0;          // superblocks
     int ntasks = 0;       // superblock pairs A < B
-    int nfull = 0;        // of them, pairs without a partial superblock (launched first)
+    int split = 1;        // workgroups per task
     size_t ipart_off = 0, jpart_off = 0, dpart_off = 0, tasks_off = 0, bytes = 0;   // workspace layout (bytes)
 };
+
+// Workgroups per task: the pair loop of a task takes about 223 us on a CU (its
+// SIMDs are issue-bound from one wavefront on, so two workgroups on a CU take twice
+// that), and every part writes and the reduction reads 24 KB of target-side
+// sums, about 12 ns of the chip's bandwidth.  The split with the least
+// modelled time; measured (leapfrog steps, FP64): 8192 bodies 59 us (286
+// unsplit), 10007 75 (526), 20000 210 (566), 24576 301 (513), 49152 965 (1200).
+static int sym_split(int ntasks) {
+    constexpr int kCUs = 256;
+    constexpr double kTask = 223., kPart = 0.012;   // us
+    int best = 1;
+    double least = 1e300;
+    for (int s = 1; s <= kSymSB / kSymJB; s *= 2) {
+        const double t = (ntasks * s + kCUs - 1) / kCUs * kTask / s + ntasks * s * kPart;
+        if (t < least) {
+            least = t;
+            best = s;
+        }
+    }
+    return best;
+}
 
 static SymPlan sym_plan(int N) {
     SymPlan p;
     p.nsb = (N + kSymSB - 1) / kSymSB;
     p.ntasks = p.nsb * (p.nsb - 1) / 2;
-    const bool ragged = N % kSymSB != 0;
-    p.nfull = ragged ? (p.nsb - 1) * (p.nsb - 2) / 2 : p.ntasks;
+    p.split = sym_split(p.ntasks);
     const size_t part = sizeof(double) * 3 * (size_t)kSymSB * (size_t)p.ntasks;
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.ipart_off = 0;
-    p.jpart_off = up(part);
+    p.jpart_off = up(part * p.split);
     p.dpart_off = p.jpart_off + up(part);
-    p.tasks_off = p.dpart_off + up(sizeof(double) * 6 * (size_t)N);
+    p.tasks_off = p.dpart_off + up(sizeof(double) * 6 * kSymDiag * (size_t)N);
     p.bytes = p.tasks_off + up(sizeof(int2) * (size_t)(p.ntasks > 0 ? p.ntasks : 1));
     return p;
 }
 
-// The task list (A, B), A < B: pairs without the ragged last superblock first,
-// then those with it (launched with the bounds checks).
+// The task list (A, B), A < B.
 static std::vector<int2> sym_tasks(const SymPlan& p) {
     std::vector<int2> t;
     t.reserve(p.ntasks);
-    const int last = (p.nfull == p.ntasks) ? p.nsb : p.nsb - 1;
-    for (int A = 0; A < last; A++)
-        for (int B = A + 1; B < last; B++) t.push_back(make_int2(A, B));
-    if (last < p.nsb)
-        for (int A = 0; A < last; A++) t.push_back(make_int2(A, last));
+    for (int A = 0; A < p.nsb; A++)
+        for (int B = A + 1; B < p.nsb; B++) t.push_back(make_int2(A, B));
     return t;
 }
 
@@ -990,16 +1059,14 @@ bool gravity_symmetric_path(size_t N, int precision, bool compensated) {
 }
 size_t gravity_symmetric_bytes(size_t N) { return sym_plan((int)N).bytes; }
 
-// Ordered pairs inside the superblocks (evaluated by k_direct_diag, not by
-// the symmetric kernel): sum over superblocks of n_A^2, self pairs included.
+// Ordered pairs inside the superblocks (evaluated one-sided): sum over superblocks of n_A^2, self pairs included.
 static double sym_diag_pairs(int N) {
     const int full = N / kSymSB, rest = N % kSymSB;
     return (double)full * kSymSB * kSymSB + (double)rest * rest;
 }
 
-// One force evaluation on the symmetric path: the pairs inside superblocks,
-// the superblock pairs (events around these), then the per-body reduction
-// with the fused kick and drift.
+// One force evaluation on the symmetric path: all pairs (events around this
+// launch), then the per-body reduction with the fused kick and drift.
 static int sym_launch(int mode, const double* x, const double* y, const double* z, const double* m, double* ax,
                       double* ay, double* az, int N, double G, double soft2, const SymPlan& plan, char* base,
                       hipStream_t st, hipEvent_t* ev, const KickDrift& kd) {
@@ -1007,32 +1074,17 @@ static int sym_launch(int mode, const double* x, const double* y, const double* 
     double* jpart = reinterpret_cast<double*>(base + plan.jpart_off);
     double* dpart = reinterpret_cast<double*>(base + plan.dpart_off);
     const int2* tasks = reinterpret_cast<const int2*>(base + plan.tasks_off);
-    const dim3 gdiag(plan.nsb * (kSymSB / kFast));
-    if (mode == FM_SPLIT)
-        hipLaunchKernelGGL(k_direct_diag<FM_SPLIT>, gdiag, dim3(kFast), 0, st, x, y, z, m, N, soft2, dpart);
-    else
-        hipLaunchKernelGGL(k_direct_diag<FM_FP64>, gdiag, dim3(kFast), 0, st, x, y, z, m, N, soft2, dpart);
+    const dim3 grid(plan.ntasks * plan.split + (N + kFast - 1) / kFast * kSymDiag);
     if (ev) (void)hipEventRecord(ev[0], st);
-    const int nrag = plan.ntasks - plan.nfull;
-    if (plan.nfull > 0) {
-        if (mode == FM_SPLIT)
-            hipLaunchKernelGGL((k_direct_sym<FM_SPLIT, false>), dim3(plan.nfull), dim3(256), 0, st, x, y, z, m, N,
-                               plan.nsb, soft2, tasks, 0, ipart, jpart);
-        else
-            hipLaunchKernelGGL((k_direct_sym<FM_FP64, false>), dim3(plan.nfull), dim3(256), 0, st, x, y, z, m, N,
-                               plan.nsb, soft2, tasks, 0, ipart, jpart);
-    }
-    if (nrag > 0) {
-        if (mode == FM_SPLIT)
-            hipLaunchKernelGGL((k_direct_sym<FM_SPLIT, true>), dim3(nrag), dim3(256), 0, st, x, y, z, m, N,
-                               plan.nsb, soft2, tasks, plan.nfull, ipart, jpart);
-        else
-            hipLaunchKernelGGL((k_direct_sym<FM_FP64, true>), dim3(nrag), dim3(256), 0, st, x, y, z, m, N,
-                               plan.nsb, soft2, tasks, plan.nfull, ipart, jpart);
-    }
+    if (mode == FM_SPLIT)
+        hipLaunchKernelGGL(k_direct_sym<FM_SPLIT>, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks,
+                           plan.split, soft2, tasks, ipart, jpart, dpart);
+    else
+        hipLaunchKernelGGL(k_direct_sym<FM_FP64>, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks,
+                           plan.split, soft2, tasks, ipart, jpart, dpart);
     if (ev) (void)hipEventRecord(ev[1], st);
-    hipLaunchKernelGGL(k_sym_reduce, dim3((N + 255) / 256), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb, -G,
-                       ax, ay, az, kd);
+    hipLaunchKernelGGL(k_sym_reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb,
+                       plan.split, -G, ax, ay, az, kd);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
