@@ -13,6 +13,8 @@
 
 using namespace rbamd;
 
+extern "C" void rb_whfast_step(struct reb_simulation* r, void* state);
+
 static volatile sig_atomic_t g_sigint = 0;
 static void sigint_handler(int signum) {
     if (signum == SIGINT) g_sigint += 1;
@@ -105,6 +107,51 @@ static bool builtin_device_integrator(const struct reb_simulation* r) {
     return n && (strcmp(n, "leapfrog") == 0 || strcmp(n, "sei") == 0 || strcmp(n, "whfast") == 0);
 }
 
+static void count_steps(struct reb_simulation* const r, const struct timeval& t0, size_t n) {
+    struct timeval t1;
+    gettimeofday(&t1, nullptr);
+    const double elapsed = t1.tv_sec - t0.tv_sec + (t1.tv_usec - t0.tv_usec) / 1e6;
+    r->walltime_last_step = elapsed / (double)n;
+    r->walltime_last_steps_sum += elapsed;
+    r->walltime_last_steps_N += (int)n;
+    if (r->walltime_last_steps_sum > 0.1) {
+        r->walltime_last_steps = r->walltime_last_steps_sum / r->walltime_last_steps_N;
+        r->walltime_last_steps_sum = 0;
+        r->walltime_last_steps_N = 0;
+    }
+    r->walltime += elapsed;
+    r->steps_done += n;
+}
+
+// Whether nothing on the host looks at the simulation between its WHFast
+// steps, so that several can run in one launch: no callback, exit check,
+// boundary, collision search, archive or variational set (whose rescaling and
+// MEGNO sums are formed on the host after every step).
+static bool steps_unobserved(const struct reb_simulation* r) {
+    return r->integrator.callbacks.step == rb_whfast_step && !r->heartbeat && !r->pre_timestep_modifications &&
+           !r->post_timestep_modifications && !r->additional_forces && !r->exit_max_distance &&
+           !r->exit_min_distance && !r->simulationarchive_filename && r->boundary == REB_BOUNDARY_NONE &&
+           r->collision == REB_COLLISION_NONE && !r->N_odes && !r->N_var && r->usleep <= 0;
+}
+
+// A launch holds at most this many steps (about 10 ms), so that an interrupt is
+// seen soon.
+static constexpr size_t kLaunchSteps = 1000;
+
+// Up to n <= kLaunchSteps steps in one launch; one launch per step (metadata
+// copies, two waits, two launches) cost 40 us for an 8-planet system whose step
+// takes 9 us on the device.  Returns the steps done, 0 when the caller has to
+// step one by one.  A refused launch counts as one step, as a refused step does.
+static size_t whfast_steps_at_once(struct reb_simulation* const r, size_t n) {
+    if (n < 2 || !steps_unobserved(r)) return 0;
+    struct timeval t0;
+    gettimeofday(&t0, nullptr);
+    if (!whfast_steps_device(r, (struct reb_integrator_whfast_state*)r->integrator.state, (long)n)) n = 1;
+    r->did_modify_particles = 0;
+    count_steps(r, t0, n);
+    return n;
+}
+
 // simulation.c:514-603
 static void reb_simulation_step(struct reb_simulation* const r) {
     struct timeval t0;
@@ -141,18 +188,7 @@ static void reb_simulation_step(struct reb_simulation* const r) {
         if (collision_search_device(r)) collision_resolve_host(r);
     }
     (void)d;
-    struct timeval t1;
-    gettimeofday(&t1, nullptr);
-    r->walltime_last_step = t1.tv_sec - t0.tv_sec + (t1.tv_usec - t0.tv_usec) / 1e6;
-    r->walltime_last_steps_sum += r->walltime_last_step;
-    r->walltime_last_steps_N += 1;
-    if (r->walltime_last_steps_sum > 0.1) {
-        r->walltime_last_steps = r->walltime_last_steps_sum / r->walltime_last_steps_N;
-        r->walltime_last_steps_sum = 0;
-        r->walltime_last_steps_N = 0;
-    }
-    r->walltime += r->walltime_last_step;
-    r->steps_done++;
+    count_steps(r, t0, 1);
 }
 
 // simulation.c:291-369
@@ -204,6 +240,25 @@ static int reb_check_exit(struct reb_simulation* const r, const double tmax, dou
     return r->status;
 }
 
+// Steps of the present dt until reb_check_exit would do more than go on, with
+// the time advanced as the steps advance it; at most kLaunchSteps.
+static size_t steps_before_exit(const struct reb_simulation* r, double tmax) {
+    if (r->status != REB_STATUS_RUNNING) return 0;
+    const double sign = copysign(1., r->dt);
+    double t = r->t;
+    size_t n = 0;
+    while (n < kLaunchSteps) {
+        if (tmax != INFINITY) {
+            const double ahead = r->exact_finish_time == 1 ? t + r->dt : t;
+            if (ahead * sign >= tmax * sign) break;
+        }
+        t += r->dt / 2.;
+        t += r->dt / 2.;
+        n++;
+    }
+    return n;
+}
+
 static void begin_call(struct reb_simulation* r) {
     // The caller may have written r->particles since the last call (unless the
     // simulation was declared device-resident).
@@ -234,6 +289,11 @@ REB_API void reb_simulation_steps(struct reb_simulation* const r, size_t N_steps
     begin_call(r);
     run_heartbeat(r);
     for (size_t i = 0; i < N_steps; i++) {
+        const size_t k = whfast_steps_at_once(r, N_steps - i < kLaunchSteps ? N_steps - i : kLaunchSteps);
+        if (k) {
+            i += k - 1;
+            continue;
+        }
         if (r->simulationarchive_filename) archive_heartbeat(r);
         reb_simulation_step(r);
         run_heartbeat(r);
@@ -266,6 +326,11 @@ REB_API enum REB_STATUS reb_simulation_integrate(struct reb_simulation* const r,
     if (r->status != REB_STATUS_PAUSED && r->status != REB_STATUS_SCREENSHOT) r->status = REB_STATUS_RUNNING;
     run_heartbeat(r);
     while (reb_check_exit(r, tmax, &last_full_dt) < 0) {
+        const size_t k = whfast_steps_at_once(r, steps_before_exit(r, tmax));
+        if (k) {
+            if (g_sigint) r->status = REB_STATUS_SIGINT;
+            continue;
+        }
         if (r->simulationarchive_filename) archive_heartbeat(r);
         reb_simulation_step(r);
         run_heartbeat(r);

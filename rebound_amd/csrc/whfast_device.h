@@ -83,6 +83,8 @@ int whfast_launch(const WHParams& P, hipStream_t st);
 bool whfast_lane_takes(const WHParams& P);
 void whfast_lane_launch(const WHParams& P, hipStream_t st);
 int whfast_lane_per_cu();
+// The general kernels (whfast_general.hip).
+void whfast_general_launch(const WHParams& P, hipStream_t st);
 int whfast_energy_launch(const WHParams& P, double* out, int nsys, hipStream_t st);
 int whfast_group_size(int K);
 int whfast_max_resident(int device);
