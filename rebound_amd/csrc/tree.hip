@@ -34,6 +34,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "ieee_mid.h"
 #include "internal.h"
 
 namespace rbamd {
@@ -62,11 +63,13 @@ struct TreeBuffers {
     DevBuf lcp, cnt, base;                        // per body
     DevBuf prim_tmp;                              // rocPRIM temporary storage
     DevBuf node_d;                                // 8 doubles per cell: cx cy cz w m mx my mz
-    DevBuf node_i;                                // 4 ints per cell: next pt level start
+    DevBuf node_i;                                // 3 ints per cell: next pt level
     DevBuf info;                                  // total, maxlevel, flags
     DevBuf coll_cnt, coll_off, coll_rec;          // collision search
     DevBuf coll_slot;                             // kCollSlots records per body (single-pass search)
     DevBuf grec, crec;                            // 64-byte walk records per cell (gravity, collisions)
+    DevBuf roots;                                 // cell of each root box, -1 if empty
+    DevBuf root_rec;                              // their records (gravity)
     size_t body_cap = 0, node_cap = 0, rec_cap = 0;
     int nnodes = 0;
     int maxlevel = 0;
@@ -112,8 +115,10 @@ __device__ __forceinline__ void descend(int o, double& cx, double& cy, double& c
 // flags: bit0 outside box, bit1 non-finite, bit2 unresolved at max depth, bit3 identical positions
 __global__ void k_tree_keys(const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
                             int n, TreeGeom g, int with_word1, unsigned long long* __restrict__ key0,
-                            unsigned long long* __restrict__ key1, int* __restrict__ idx, int* __restrict__ info) {
+                            unsigned long long* __restrict__ key1, int* __restrict__ idx, int* __restrict__ info,
+                            int* __restrict__ roots, int nroot) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int q = i; q < nroot; q += gridDim.x * blockDim.x) roots[q] = -1;   // set by k_tree_nodes
     if (i >= n) return;
     const double px = x[i], py = y[i], pz = z[i];
     idx[i] = i;
@@ -198,19 +203,29 @@ __global__ void k_tree_lcp(const unsigned long long* __restrict__ k0, const unsi
     lcp[s] = l;
 }
 
-__global__ void k_tree_count(const int* __restrict__ lcp, int n, int* __restrict__ cnt, int* __restrict__ info) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
+__global__ __launch_bounds__(256) void k_tree_count(const int* __restrict__ lcp, int n, int* __restrict__ cnt, int* __restrict__ info) {
+    const int at = blockIdx.x * blockDim.x + threadIdx.x;
+    const int s = at < n ? at : n - 1;             // every lane takes part in the reduction
     const int prev = s > 0 ? lcp[s - 1] : -1;
     const int cur = lcp[s];
     const int nint = cur > prev ? cur - prev : 0;
     cnt[s] = nint + 1;
-    atomicMax(&info[1], (prev > cur ? prev : cur) + 1);
+    // the deepest level: one atomic per workgroup (one per body took 39 us for
+    // 200000 bodies, all on one address)
+    __shared__ int deepest[4];
+    int level = (prev > cur ? prev : cur) + 1;
+    for (int off = 32; off > 0; off >>= 1) level = max(level, __shfl_xor(level, off));
+    if ((threadIdx.x & 63) == 0) deepest[threadIdx.x >> 6] = level;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        level = max(max(deepest[0], deepest[1]), max(deepest[2], deepest[3]));
+        if (level > info[1]) atomicMax(&info[1], level);
+    }
 }
 
 struct NodeArrays {
     double *cx, *cy, *cz, *w, *m, *mx, *my, *mz;
-    int *next, *pt, *level, *start;
+    int *next, *pt, *level;
 };
 
 __device__ __forceinline__ NodeArrays node_arrays(double* d, int* ii, size_t cap) {
@@ -226,7 +241,6 @@ __device__ __forceinline__ NodeArrays node_arrays(double* d, int* ii, size_t cap
     A.next = ii;
     A.pt = ii + cap;
     A.level = ii + 2 * cap;
-    A.start = ii + 3 * cap;
     return A;
 }
 
@@ -250,7 +264,7 @@ __global__ void k_tree_nodes(const unsigned long long* __restrict__ k0, const un
                              const int* __restrict__ idx, const int* __restrict__ lcp, const int* __restrict__ base,
                              int n, int total, TreeGeom g, int two, double* __restrict__ nd, int* __restrict__ ni,
                              size_t cap, const double* __restrict__ pm, const double* __restrict__ px,
-                             const double* __restrict__ py, const double* __restrict__ pz) {
+                             const double* __restrict__ py, const double* __restrict__ pz, int* __restrict__ roots) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     NodeArrays A = node_arrays(nd, ni, cap);
@@ -289,7 +303,7 @@ __global__ void k_tree_nodes(const unsigned long long* __restrict__ k0, const un
         A.next[id] = (e + 1 < n) ? base[e + 1] : total;
         A.pt[id] = -(e - s + 1);
         A.level[id] = d;
-        A.start[id] = s;
+        if (d == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
         double cx, cy, cz, w;
         cell_geometry(g, a0, a1, d, cx, cy, cz, w);
         A.cx[id] = cx;
@@ -303,7 +317,7 @@ __global__ void k_tree_nodes(const unsigned long long* __restrict__ k0, const un
     A.next[id] = id + 1;
     A.pt[id] = p;
     A.level[id] = leaf_level;
-    A.start[id] = s;
+    if (leaf_level == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
     double cx, cy, cz, w;
     cell_geometry(g, a0, a1, leaf_level, cx, cy, cz, w);
     A.cx[id] = cx;
@@ -352,6 +366,13 @@ struct __align__(64) GravRec {
     int next, pt;
     double pad;
 };
+// A root box's cell: w2 the width squared, infinite for a leaf (which is always
+// walked); its cells are first .. end - 1.
+struct __align__(16) RootRec {
+    double x, y, z, m;
+    double w2;
+    int first, end;
+};
 // A cell's record for the collision walk.  Inner cell (pt < 0): its
 // geometric centre and width.  Leaf (pt >= 0): its body's x, y, z and radius
 // in cx, cy, cz, w and its velocity in v, copied when the tree is built (the
@@ -363,28 +384,56 @@ struct __align__(64) CollCell {
     double v[3];
 };
 
-__global__ void k_tree_pack(const double* __restrict__ nd, const int* __restrict__ ni, size_t cap, int total,
-                            GravRec* __restrict__ g, CollCell* __restrict__ cc, const double* __restrict__ x,
-                            const double* __restrict__ y, const double* __restrict__ z,
-                            const double* __restrict__ vx, const double* __restrict__ vy,
-                            const double* __restrict__ vz, const double* __restrict__ rad) {
+// The walk records of all cells.  The first wavefront also writes the root
+// boxes' cells, empty boxes left out, their number, and up to three massless
+// cells far away behind them (accepted by every body, without effect), so that
+// the walk can read them in fours.
+__global__ void k_tree_pack_gravity(const double* __restrict__ nd, const int* __restrict__ ni, size_t cap, int total,
+                                    GravRec* __restrict__ g, const int* __restrict__ roots, int nroot,
+                                    RootRec* __restrict__ rr, int* __restrict__ nroots) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    auto rec = [&](int k) {
+        GravRec a;
+        a.mx = nd[5 * cap + k];
+        a.my = nd[6 * cap + k];
+        a.mz = nd[7 * cap + k];
+        a.m = nd[4 * cap + k];
+        a.w = nd[3 * cap + k];
+        a.next = ni[k];
+        a.pt = ni[cap + k];
+        a.pad = 0.;
+        return a;
+    };
+    if (c < 64) {
+        int nr = 0;
+        for (int q = 0; q < nroot; q += 64) {
+            const int id = q + c < nroot ? roots[q + c] : -1;
+            const unsigned long long have = __ballot(id >= 0);
+            if (id >= 0) {
+                const GravRec a = rec(id);
+                rr[nr + __popcll(have & ((1ull << c) - 1ull))] =
+                    RootRec{a.mx, a.my, a.mz, a.m, a.pt < 0 ? a.w * a.w : __builtin_inf(), id, a.next};
+            }
+            nr += __popcll(have);
+        }
+        if (c < 3) rr[nr + c] = RootRec{0x1p66, 0., 0., 0., 0., 0, 0};
+        if (c == 0) *nroots = nr;
+    }
+    if (c < total) g[c] = rec(c);
+}
+
+__global__ void k_tree_pack_collide(const double* __restrict__ nd, const int* __restrict__ ni, size_t cap, int total,
+                                    CollCell* __restrict__ cc, const double* __restrict__ x,
+                                    const double* __restrict__ y, const double* __restrict__ z,
+                                    const double* __restrict__ vx, const double* __restrict__ vy,
+                                    const double* __restrict__ vz, const double* __restrict__ rad) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= total) return;
-    GravRec a;
-    a.mx = nd[5 * cap + c];
-    a.my = nd[6 * cap + c];
-    a.mz = nd[7 * cap + c];
-    a.m = nd[4 * cap + c];
-    a.w = nd[3 * cap + c];
-    a.next = ni[c];
-    a.pt = ni[cap + c];
-    a.pad = 0.;
-    g[c] = a;
     CollCell b;
-    b.next = a.next;
-    b.pt = a.pt;
-    if (a.pt >= 0) {
-        const int p = a.pt;
+    b.next = ni[c];
+    b.pt = ni[cap + c];
+    if (b.pt >= 0) {
+        const int p = b.pt;
         b.cx = x[p];
         b.cy = y[p];
         b.cz = z[p];
@@ -396,7 +445,7 @@ __global__ void k_tree_pack(const double* __restrict__ nd, const int* __restrict
         b.cx = nd[c];
         b.cy = nd[cap + c];
         b.cz = nd[2 * cap + c];
-        b.w = a.w;
+        b.w = nd[3 * cap + c];
         b.v[0] = b.v[1] = b.v[2] = 0.;
     }
     cc[c] = b;
@@ -472,8 +521,12 @@ static bool tree_sort(struct reb_simulation* r, TreeBuffers* T, int n, bool two)
     return RB_HIP(r, hipGetLastError());
 }
 
-// Builds the tree of the current device positions.  tree.c:254-271 + :147-229.
-bool tree_build(struct reb_simulation* r) {
+// Builds the tree of the current device positions (tree.c:254-271): for gravity
+// with the moments (:147-229) and the gravity walk's records, for the collision
+// search with its own records (its tests read no moments, which take a launch per
+// level).
+enum TreeFor { TREE_GRAVITY, TREE_COLLISIONS };
+bool tree_build(struct reb_simulation* r, TreeFor what) {
     DeviceState* d = dev_of(r);
     if (r->root_size <= 0.0) {
         reb_simulation_error(r, "Set root_size to a finite value to use a tree based gravity or collision solver.");
@@ -484,6 +537,10 @@ bool tree_build(struct reb_simulation* r) {
     const int n = (int)r->N;
     if (!tree_alloc(r, T, n ? n : 1)) return false;
     TreeGeom g = tree_geom(r, T);
+    if (!T->roots.ensure(sizeof(int) * (size_t)T->nroot)) {
+        reb_simulation_error(r, "Out of device memory for the tree.");
+        return false;
+    }
     int* info = T->info.as<int>();
     bool two = false;
     int hinfo[4] = {0, 0, 0, 0};
@@ -494,7 +551,7 @@ bool tree_build(struct reb_simulation* r) {
         if (n == 0) break;
         hipLaunchKernelGGL(k_tree_keys, dim3((n + 255) / 256), dim3(256), 0, d->stream, d->field(FX), d->field(FY),
                            d->field(FZ), n, g, two ? 1 : 0, T->key0.as<unsigned long long>(),
-                           T->key1.as<unsigned long long>(), T->idx.as<int>(), info);
+                           T->key1.as<unsigned long long>(), T->idx.as<int>(), info, T->roots.as<int>(), T->nroot);
         if (!tree_sort(r, T, n, two)) return false;
         hipLaunchKernelGGL(k_tree_lcp, dim3((n + 255) / 256), dim3(256), 0, d->stream,
                            T->key0.as<unsigned long long>(), T->key1.as<unsigned long long>(), n, g.L1, g.L2,
@@ -540,7 +597,7 @@ bool tree_build(struct reb_simulation* r) {
     if ((size_t)total > T->node_cap) {
         size_t cap = T->node_cap ? T->node_cap : 4096;
         while (cap < (size_t)total) cap *= 2;
-        if (!T->node_d.ensure(sizeof(double) * 8 * cap) || !T->node_i.ensure(sizeof(int) * 4 * cap)) {
+        if (!T->node_d.ensure(sizeof(double) * 8 * cap) || !T->node_i.ensure(sizeof(int) * 3 * cap)) {
             reb_simulation_error(r, "Out of device memory for the tree cells.");
             return false;
         }
@@ -550,43 +607,93 @@ bool tree_build(struct reb_simulation* r) {
     hipLaunchKernelGGL(k_tree_nodes, dim3((n + 255) / 256), dim3(256), 0, d->stream,
                        T->key0.as<unsigned long long>(), T->key1.as<unsigned long long>(), T->idx.as<int>(),
                        T->lcp.as<int>(), T->base.as<int>(), n, total, g, two ? 1 : 0, T->node_d.as<double>(),
-                       T->node_i.as<int>(), T->node_cap, d->field(FM), d->field(FX), d->field(FY), d->field(FZ));
-    for (int lev = T->maxlevel; lev >= 0; lev--)
-        hipLaunchKernelGGL(k_tree_moments, dim3((total + 255) / 256), dim3(256), 0, d->stream,
-                           T->node_d.as<double>(), T->node_i.as<int>(), T->node_cap, total, lev);
-    if (!T->grec.ensure(sizeof(GravRec) * (size_t)total) || !T->crec.ensure(sizeof(CollCell) * (size_t)total)) {
+                       T->node_i.as<int>(), T->node_cap, d->field(FM), d->field(FX), d->field(FY), d->field(FZ),
+                       T->roots.as<int>());
+    const dim3 cells((total + 255) / 256);
+    if (!(what == TREE_GRAVITY ? T->grec.ensure(sizeof(GravRec) * (size_t)total) &&
+                                     T->root_rec.ensure(sizeof(RootRec) * ((size_t)T->nroot + 3))
+                               : T->crec.ensure(sizeof(CollCell) * (size_t)total))) {
         reb_simulation_error(r, "Out of device memory for the tree cells.");
         return false;
     }
-    hipLaunchKernelGGL(k_tree_pack, dim3((total + 255) / 256), dim3(256), 0, d->stream, T->node_d.as<double>(),
-                       T->node_i.as<int>(), T->node_cap, total, T->grec.as<GravRec>(), T->crec.as<CollCell>(),
-                       d->field(FX), d->field(FY), d->field(FZ), d->field(FVX), d->field(FVY), d->field(FVZ),
-                       d->field(FR));
+    if (what == TREE_GRAVITY) {
+        for (int lev = T->maxlevel; lev >= 0; lev--)
+            hipLaunchKernelGGL(k_tree_moments, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
+                               T->node_i.as<int>(), T->node_cap, total, lev);
+        hipLaunchKernelGGL(k_tree_pack_gravity, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
+                           T->node_i.as<int>(), T->node_cap, total, T->grec.as<GravRec>(), T->roots.as<int>(),
+                           T->nroot, T->root_rec.as<RootRec>(), info + 3);
+    } else {
+        hipLaunchKernelGGL(k_tree_pack_collide, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
+                           T->node_i.as<int>(), T->node_cap, total, T->crec.as<CollCell>(), d->field(FX), d->field(FY),
+                           d->field(FZ), d->field(FVX), d->field(FVY), d->field(FVZ), d->field(FR));
+    }
     return RB_HIP(r, hipGetLastError());
 }
 
 // ---------------------------------------------------------------- tree gravity
+// Workgroups go to the 8 XCDs in turn; block b of nb takes piece (b % 8) of the
+// key order, so that the bodies of one XCD are neighbours and share the tree
+// cells in its L2.
+static constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_block() {
+    const int per = (int)gridDim.x / kXcds;          // the grid is a multiple of kXcds
+    return ((int)blockIdx.x % kXcds) * per + (int)blockIdx.x / kXcds;
+}
+static dim3 xcd_grid(int blocks) { return dim3((blocks + kXcds - 1) / kXcds * kXcds); }
+
+// Bodies per wavefront of a walk.  A wavefront walks the union of its bodies'
+// cells, so 64 give the least work; with fewer wavefronts than half the SIMDs the
+// length of one walk sets the time, which fewer bodies shorten (12007 bodies, a
+// step with tree gravity: 763 us with 32 bodies, 680 with 16; 30000: 968 with 64,
+// 934 with 32, 1001 with 16; 60000: 1275 with 64, 1375 with 32).
+static constexpr int kWalkWaves = 512;
+static int walk_bodies(int n) {
+    int w = 64;
+    while (w > 8 && (n + w - 1) / w < kWalkWaves) w /= 2;
+    return w;
+}
+
 // tree.c:275-328 for every ghost box (gravity.c:84-102), in the reference's
-// expressions; 64 bodies (in key order) per wavefront.
+// expressions; `width` bodies (in key order) per wavefront.
+//
+// Most of a body's terms are whole root boxes (200000 bodies in 100 root boxes
+// with 25 images: 2500 of 2855).  The wavefront reads their records four at a
+// time from a table (uniform, in the scalar cache).  Four that no lane opens are
+// evaluated together, four independent square root and division chains, and added in
+// order; a root box that some lane opens is walked along the pre-order, cell by
+// cell.  The square roots and divisions are the short sequences of
+// ieee_mid.h, or the compiler's if an operand is out of their range.  200000
+// bodies: 2.43 ms one cell at a time, now 1.9; what bounds it is the latency of the
+// near part's cell fetches and the FP64 issue of the wavefronts of the SIMDs that hold
+// four (3125 wavefronts on 1024 SIMDs).
 __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__ rec, int total,
-                                                     const int* __restrict__ idx, int n,
-                                                     const double* __restrict__ x, const double* __restrict__ y,
-                                                     const double* __restrict__ z, GBT gl, double G, double soft2,
-                                                     double theta2, double* __restrict__ ax,
-                                                     double* __restrict__ ay, double* __restrict__ az,
+                                                     const RootRec* __restrict__ root,
+                                                     const int* __restrict__ nroots, const int* __restrict__ idx,
+                                                     int n, int width, const double* __restrict__ x,
+                                                     const double* __restrict__ y, const double* __restrict__ z,
+                                                     GBT gl, double G, double soft2, double theta2,
+                                                     double* __restrict__ ax, double* __restrict__ ay,
+                                                     double* __restrict__ az,
                                                      unsigned long long* __restrict__ counter) {
-    const int s = blockIdx.x * 64 + threadIdx.x;
-    const bool live = s < n;
+    const int lane = threadIdx.x;
+    const int s = xcd_block() * width + lane;
+    if (s - lane >= n) return;                       // one wave per block: uniform
+    const bool live = lane < width && s < n;
     const int me = live ? idx[s] : -1;
-    const double xi = live ? x[me] : 0., yi = live ? y[me] : 0., zi = live ? z[me] : 0.;
+    // lanes without a body sit at the wavefront's first body: they open nothing
+    // that it does not open, and their sums are not stored
+    const int src = idx[live ? s : s - lane];
+    const double xi = x[src], yi = y[src], zi = z[src];
     double a_x = 0., a_y = 0., a_z = 0.;
-    unsigned long long inter = 0;
-    for (int g = 0; g < gl.n; g++) {
-        const double gx = gl.g[g][0] + xi, gy = gl.g[g][1] + yi, gz = gl.g[g][2] + zi;
+    unsigned int inter = 0;
+    const int nr = *nroots;
+    const bool g_mid = mid_distance(fabs(G)) < kMidSpan;
+    // cells c .. end - 1 in pre-order
+    auto walk = [&](int c, int end, double gx, double gy, double gz) {
         int skip = live ? 0 : 0x7fffffff;
-        int c = 0;
-        GravRec cur = rec[0];
-        while (c < total) {
+        GravRec cur = rec[c];
+        while (c < end) {
             // both possible successors are fetched before this cell is evaluated
             const int c_open = c + 1, c_skip = cur.next;
             const GravRec r_open = rec[c_open < total ? c_open : total - 1];
@@ -611,8 +718,16 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                     use = false;
                 }
                 if (use) {
-                    const double _r = sqrt(r2 + soft2);
-                    const double prefact = -G / (_r * _r * _r) * cur.m;
+                    const double rs = r2 + soft2;
+                    double f;
+                    if (g_mid && mid_distance(rs) < kMidSpan) {
+                        const double _r = sqrt_mid(rs);
+                        f = div_mid(-G, _r * _r * _r);
+                    } else {
+                        const double _r = sqrt(rs);
+                        f = -G / (_r * _r * _r);
+                    }
+                    const double prefact = f * cur.m;
                     a_x += prefact * dx;
                     a_y += prefact * dy;
                     a_z += prefact * dz;
@@ -623,6 +738,61 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
             c = any ? c_open : c_skip;
             cur = any ? r_open : r_skip;
         }
+    };
+    for (int g = 0; g < gl.n; g++) {
+        const double gx = gl.g[g][0] + xi, gy = gl.g[g][1] + yi, gz = gl.g[g][2] + zi;
+        for (int k = 0; k < nr; k += 4) {
+            RootRec c[4];
+            double dx[4], dy[4], dz[4], r2[4], f[4];
+            unsigned long long open[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) c[q] = root[k + q];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                dx[q] = gx - c[q].x;
+                dy[q] = gy - c[q].y;
+                dz[q] = gz - c[q].z;
+                r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
+                open[q] = __ballot(c[q].w2 > theta2 * r2[q]);
+            }
+            unsigned int far = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const double rs = r2[q] + soft2;
+                far = max(far, mid_distance(rs));
+                const double _r = sqrt_mid(rs);
+                f[q] = div_mid(-G, _r * _r * _r) * c[q].m;
+            }
+            if (!g_mid || __any(far >= kMidSpan)) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const double _r = sqrt(r2[q] + soft2);
+                    f[q] = -G / (_r * _r * _r) * c[q].m;
+                }
+            }
+            if ((open[0] | open[1] | open[2] | open[3]) == 0ull) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    a_x += f[q] * dx[q];
+                    a_y += f[q] * dy[q];
+                    a_z += f[q] * dz[q];
+                }
+                inter += min(4, nr - k);
+                continue;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (k + q >= nr) break;
+                if (open[q]) {
+                    walk(c[q].first, c[q].end, gx, gy, gz);
+                } else {
+                    a_x += f[q] * dx[q];
+                    a_y += f[q] * dy[q];
+                    a_z += f[q] * dz[q];
+                    inter++;
+                }
+            }
+        }
     }
     if (live) {
         ax[me] = a_x;
@@ -631,8 +801,9 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
     }
     if (counter) {
         // per-wave reduction of the interaction count
-        for (int off = 32; off > 0; off >>= 1) inter += __shfl_down(inter, off);
-        if (threadIdx.x == 0) atomicAdd(counter, inter);
+        unsigned long long sum = live ? inter : 0;
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off);
+        if (threadIdx.x == 0) atomicAdd(counter, sum);
     }
 }
 
@@ -640,7 +811,7 @@ bool gravity_tree(struct reb_simulation* r) {
     DeviceState* d = dev_of(r);
     // gravity.c:54-56: wrap into the box before building
     if (!boundary_device(r)) return false;
-    if (!tree_build(r)) return false;
+    if (!tree_build(r, TREE_GRAVITY)) return false;
     TreeBuffers* T = d->tree;
     const int n = (int)r->N;
     if (n == 0) return true;
@@ -661,10 +832,12 @@ bool gravity_tree(struct reb_simulation* r) {
     }
     unsigned long long* counter = reinterpret_cast<unsigned long long*>(T->info.as<int>() + 8);
     if (!RB_HIP(r, hipMemsetAsync(counter, 0, 8, d->stream))) return false;
-    hipLaunchKernelGGL(k_tree_gravity, dim3((n + 63) / 64), dim3(64), 0, d->stream, T->grec.as<GravRec>(),
-                       T->nnodes, T->idx.as<int>(), n, d->field(FX),
-                       d->field(FY), d->field(FZ), gl, r->G, r->softening * r->softening, r->opening_angle2,
-                       d->field(FAX), d->field(FAY), d->field(FAZ), counter);
+    const int width = walk_bodies(n);
+    const dim3 grid = xcd_grid((n + width - 1) / width);
+    hipLaunchKernelGGL(k_tree_gravity, grid, dim3(64), 0, d->stream, T->grec.as<GravRec>(), T->nnodes,
+                       T->root_rec.as<RootRec>(), T->info.as<int>() + 3, T->idx.as<int>(), n, width, d->field(FX), d->field(FY), d->field(FZ), gl, r->G,
+                       r->softening * r->softening, r->opening_angle2, d->field(FAX), d->field(FAY), d->field(FAZ),
+                       counter);
     mark_device_newer(r);
     return RB_HIP(r, hipGetLastError());
 }
@@ -672,6 +845,16 @@ bool gravity_tree(struct reb_simulation* r) {
 // ---------------------------------------------------------------- collision search
 // Largest and second-largest radius (simulation.c:718-799); only the second
 // value is used by the search.  Value-based, so independent of the order.
+// The two largest of (a1 >= a2) and (b1 >= b2).
+__device__ __forceinline__ void top2_merge(double b1, double b2, double& a1, double& a2) {
+    if (b1 > a1) {
+        a2 = a1 > b2 ? a1 : b2;
+        a1 = b1;
+    } else if (b1 > a2) {
+        a2 = b1;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_top2(const double* __restrict__ rad, int n, double* __restrict__ out) {
     __shared__ double s1[256], s2[256];
     double a1 = -1.0, a2 = -1.0;
@@ -687,39 +870,27 @@ __global__ __launch_bounds__(256) void k_top2(const double* __restrict__ rad, in
     s1[threadIdx.x] = a1;
     s2[threadIdx.x] = a2;
     __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) top2_merge(s1[threadIdx.x + w], s2[threadIdx.x + w], a1, a2);
+        s1[threadIdx.x] = a1;
+        s2[threadIdx.x] = a2;
+        __syncthreads();
+    }
     if (threadIdx.x == 0) {
-        double b1 = -1.0, b2 = -1.0;
-        for (int k = 0; k < 256; k++) {
-            const double vs[2] = {s1[k], s2[k]};
-            for (double v : vs) {
-                if (v > b1) {
-                    b2 = b1;
-                    b1 = v;
-                } else if (v > b2) {
-                    b2 = v;
-                }
-            }
-        }
-        out[2 * blockIdx.x] = b1;
-        out[2 * blockIdx.x + 1] = b2;
+        out[2 * blockIdx.x] = a1;
+        out[2 * blockIdx.x + 1] = a2;
     }
 }
 
 // The second largest radius over the blocks' top two (simulation.c:718-799),
 // left on the device for the search (0 for fewer than two bodies).
-__global__ void k_top2_final(const double* __restrict__ top, int nb, int n, double* __restrict__ second) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double b1 = -1.0, b2 = -1.0;
-    for (int k = 0; k < 2 * nb; k++) {
-        const double v = top[k];
-        if (v > b1) {
-            b2 = b1;
-            b1 = v;
-        } else if (v > b2) {
-            b2 = v;
-        }
-    }
-    *second = n >= 2 ? b2 : 0.;
+__global__ __launch_bounds__(64) void k_top2_final(const double* __restrict__ top, int nb, int n,
+                                                   double* __restrict__ second) {
+    static_assert(kTop2Blocks <= 64, "one lane per block");
+    const int lane = threadIdx.x;
+    double a1 = lane < nb ? top[2 * lane] : -1.0, a2 = lane < nb ? top[2 * lane + 1] : -1.0;
+    for (int off = 32; off > 0; off >>= 1) top2_merge(__shfl_xor(a1, off), __shfl_xor(a2, off), a1, a2);
+    if (lane == 0) *second = n >= 2 ? a2 : 0.;
 }
 
 // Swept-sphere test of LINE and LINETREE (collision.c:150-171, :510-534):
@@ -772,6 +943,14 @@ struct CollRec {
     int p1, p2, gb, ri;
 };
 
+// A root box as the collision walk's filter reads it.
+struct RootBox {
+    double x, y, z, w;
+    int first, end, leaf, pad;
+};
+
+static constexpr int kRootLds = 256;     // root boxes the filter takes (LDS)
+
 // Records kept per body by the single-pass search; the bodies with more
 // collisions are searched again by a pass that walks only them.
 static constexpr int kCollSlots = 32;
@@ -788,7 +967,8 @@ static constexpr int kCollSlots = 32;
 // drift of the last step, dt_last_done*|v|max.
 template <int MODE, bool LINE = false>
 __global__ __launch_bounds__(64) void k_tree_collide(const CollCell* __restrict__ cells, int total,
-                                                     const int* __restrict__ idx, int n,
+                                                     const int* __restrict__ idx, int n, int width,
+                                                     const int* __restrict__ roots, int nroot,
                                                      const double* __restrict__ x, const double* __restrict__ y,
                                                      const double* __restrict__ z, const double* __restrict__ vx,
                                                      const double* __restrict__ vy, const double* __restrict__ vz,
@@ -799,9 +979,13 @@ __global__ __launch_bounds__(64) void k_tree_collide(const CollCell* __restrict_
                                                      const double* __restrict__ reach_d = nullptr) {
     if (reach_d) reach = *reach_d;
     constexpr bool WRITE = MODE == 1 || MODE == 3;
-    const int s = blockIdx.x * 64 + threadIdx.x;
-    const int me = s < n ? idx[s] : -1;
-    const bool live = s < n && (MODE != 3 || counts[me] > kCollSlots);
+    extern __shared__ RootBox rootbox[];             // nroot (up to kRootLds)
+    const int lane = threadIdx.x;
+    const int s = xcd_block() * width + lane;
+    if (s - lane >= n) return;
+    const bool mine = lane < width && s < n;
+    const int me = mine ? idx[s] : -1;
+    const bool live = mine && (MODE != 3 || counts[me] > kCollSlots);
     if (MODE == 3 && __ballot(live) == 0ull) return;   // one wave per block: uniform exit
     const double px = live ? x[me] : 0., py = live ? y[me] : 0., pz = live ? z[me] : 0.;
     const double pvx = live ? vx[me] : 0., pvy = live ? vy[me] : 0., pvz = live ? vz[me] : 0.;
@@ -816,14 +1000,14 @@ __global__ __launch_bounds__(64) void k_tree_collide(const CollCell* __restrict_
         if (MODE == 2 && found < kCollSlots) slot[found] = CollRec{me, pt, g, ri};
         found++;
     };
-    for (int g = 0; g < gl.n; g++) {
+    // cells c .. end - 1 in pre-order, for ghost box g
+    auto walk = [&](int g, int c, int end) {
         const double gx = gl.g[g][0] + px, gy = gl.g[g][1] + py, gz = gl.g[g][2] + pz;
         const double gvx = gl.g[g][3] + pvx, gvy = gl.g[g][4] + pvy, gvz = gl.g[g][5] + pvz;
         int skip = live ? 0 : 0x7fffffff;
-        int c = 0;
-        int ri = -1;
-        CollCell cur = cells[0];
-        while (c < total) {
+        const int ri = -1;                           // set by k_coll_root
+        CollCell cur = cells[c];
+        while (c < end) {
             // both possible successors are fetched before this cell is evaluated
             const int c_open = c + 1, nx = cur.next;
             const CollCell r_open = cells[c_open < total ? c_open : total - 1];
@@ -867,6 +1051,60 @@ __global__ __launch_bounds__(64) void k_tree_collide(const CollCell* __restrict_
             const bool any = __ballot(open) != 0ull;
             c = any ? c_open : nx;
             cur = any ? r_open : r_skip;
+        }
+    };
+    // The root boxes that some body of the wavefront can open: a cell is opened
+    // when r2 < rp^2 with rp growing in the body's reach and r2 in its distance,
+    // so a box farther from the bodies' bounding box than the largest reach (every
+    // operation rounds monotonically) would only be tested and skipped.  Leaves
+    // are always taken.  One lane per root box instead of one visit each: of 100
+    // root boxes and 9 images a wavefront keeps about 10.
+    int nr = 0;
+    if (nroot <= kRootLds) {
+        for (int q = 0; q < nroot; q += 64) {
+            const int id = q + lane < nroot ? roots[q + lane] : -1;
+            const unsigned long long have = __ballot(id >= 0);
+            if (id >= 0) {
+                const CollCell t = cells[id];
+                rootbox[nr + __popcll(have & ((1ull << lane) - 1ull))] =
+                    RootBox{t.cx, t.cy, t.cz, t.w, id, t.next, t.pt >= 0, 0};
+            }
+            nr += __popcll(have);
+        }
+        __syncthreads();
+    }
+    const double rb = LINE ? p1_r_plus_dtv : p1_r;
+    double lo[4] = {live ? px : __builtin_inf(), live ? py : __builtin_inf(), live ? pz : __builtin_inf(),
+                    live ? rb : __builtin_inf()};
+    double hi[4] = {live ? px : -__builtin_inf(), live ? py : -__builtin_inf(), live ? pz : -__builtin_inf(),
+                    live ? rb : -__builtin_inf()};
+    for (int off = 32; off > 0; off >>= 1)
+        for (int f = 0; f < 4; f++) {
+            lo[f] = fmin(lo[f], __shfl_xor(lo[f], off));
+            hi[f] = fmax(hi[f], __shfl_xor(hi[f], off));
+        }
+    for (int g = 0; g < gl.n; g++) {
+        if (nroot > kRootLds) {
+            walk(g, 0, total);
+            continue;
+        }
+        for (int k = 0; k < nr; k += 64) {
+            bool take = false;
+            if (k + lane < nr) {
+                const RootBox t = rootbox[k + lane];
+                const double c3[3] = {t.x, t.y, t.z};
+                double d[3];
+                for (int f = 0; f < 3; f++)
+                    d[f] = fmax(fmax((gl.g[g][f] + lo[f]) - c3[f], c3[f] - (gl.g[g][f] + hi[f])), 0.);
+                const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+                const double r1 = hi[3] + reach + 0.86602540378443 * t.w;
+                const double r0 = lo[3] + reach + 0.86602540378443 * t.w;
+                take = t.leaf || !(d2 >= fmax(r1 * r1, r0 * r0));
+            }
+            for (unsigned long long left = __ballot(take); left != 0ull; left &= left - 1ull) {
+                const RootBox& t = rootbox[k + __builtin_ctzll(left)];
+                walk(g, __builtin_amdgcn_readfirstlane(t.first), __builtin_amdgcn_readfirstlane(t.end));
+            }
         }
     }
     if ((MODE == 0 || MODE == 2) && live) counts[me] = found;
@@ -1079,9 +1317,11 @@ static long tree_collide_run(struct reb_simulation* r, TreeBuffers* T, int n, co
     }
     int* overflow = T->info.as<int>() + 12;
     if (!RB_HIP(r, hipMemsetAsync(overflow, 0, sizeof(int), d->stream))) return -1;
-    const dim3 grid((n + 63) / 64);
-    hipLaunchKernelGGL((k_tree_collide<2, LINE>), grid, dim3(64), 0, d->stream, T->crec.as<CollCell>(), T->nnodes,
-                       T->idx.as<int>(), n, d->field(FX), d->field(FY), d->field(FZ), d->field(FVX), d->field(FVY),
+    const int width = walk_bodies(n);
+    const dim3 grid = xcd_grid((n + width - 1) / width);
+    const size_t lds = T->nroot <= kRootLds ? sizeof(RootBox) * (size_t)T->nroot : 0;
+    hipLaunchKernelGGL((k_tree_collide<2, LINE>), grid, dim3(64), lds, d->stream, T->crec.as<CollCell>(), T->nnodes,
+                       T->idx.as<int>(), n, width, T->roots.as<int>(), T->nroot, d->field(FX), d->field(FY), d->field(FZ), d->field(FVX), d->field(FVY),
                        d->field(FVZ), d->field(FR), gl, reach, T->coll_cnt.as<int>(), nullptr,
                        T->coll_slot.as<CollRec>(), dt_last, overflow, reach_d);
     // while the device searches: the shuffle's random draws, sized by the
@@ -1097,9 +1337,10 @@ static long tree_collide_run(struct reb_simulation* r, TreeBuffers* T, int n, co
     hipLaunchKernelGGL(k_coll_compact, dim3((n + 255) / 256), dim3(256), 0, d->stream, T->coll_cnt.as<int>(),
                        T->coll_off.as<int>(), T->coll_slot.as<CollRec>(), n, T->coll_rec.as<CollRec>());
     if (hover)
-        hipLaunchKernelGGL((k_tree_collide<3, LINE>), grid, dim3(64), 0, d->stream, T->crec.as<CollCell>(),
-                           T->nnodes, T->idx.as<int>(), n, d->field(FX), d->field(FY), d->field(FZ), d->field(FVX),
-                           d->field(FVY), d->field(FVZ), d->field(FR), gl, reach, T->coll_cnt.as<int>(),
+        hipLaunchKernelGGL((k_tree_collide<3, LINE>), grid, dim3(64), lds, d->stream, T->crec.as<CollCell>(),
+                           T->nnodes, T->idx.as<int>(), n, width, T->roots.as<int>(), T->nroot, d->field(FX),
+                           d->field(FY), d->field(FZ), d->field(FVX), d->field(FVY), d->field(FVZ), d->field(FR), gl,
+                           reach, T->coll_cnt.as<int>(),
                            T->coll_off.as<int>(), T->coll_rec.as<CollRec>(), dt_last, nullptr, reach_d);
     // root index of each record (the lcp buffer is free now: reuse as pos_of)
     int* pos_of = T->lcp.as<int>();
@@ -1155,7 +1396,7 @@ bool collision_search_device(struct reb_simulation* r) {
             return fetch_collisions(r, T, total, gl);
         }
         case REB_COLLISION_TREE: {
-            if (!tree_build(r)) return false;
+            if (!tree_build(r, TREE_COLLISIONS)) return false;
             // second largest radius, left on the device for the search
             double* top = reinterpret_cast<double*>(T->info.as<int>() + 16);
             double* second_r = top + 2 * kTop2Blocks;
@@ -1201,7 +1442,7 @@ bool collision_search_device(struct reb_simulation* r) {
             double vmax2 = 0.;
             for (double v : h) vmax2 = vmax2 > v ? vmax2 : v;
             const double maxdrift = dt_last * sqrt(vmax2);
-            if (!tree_build(r)) return false;
+            if (!tree_build(r, TREE_COLLISIONS)) return false;
             const long total = tree_collide_run<true>(r, T, n, gl, maxdrift, dt_last);
             if (total < 0) return false;
             return fetch_collisions(r, T, total, gl);
@@ -1217,7 +1458,8 @@ void tree_release(struct reb_simulation* r) {
     TreeBuffers* T = d->tree;
     for (DevBuf* b : {&T->key0, &T->key1, &T->idx, &T->key0b, &T->key1b, &T->idxb, &T->lcp, &T->cnt, &T->base,
                       &T->prim_tmp, &T->node_d, &T->node_i, &T->info, &T->coll_cnt, &T->coll_off, &T->coll_rec,
-                      &T->coll_slot, &T->grec, &T->crec})
+                      &T->coll_slot, &T->grec, &T->crec, &T->roots,
+                      &T->root_rec})
         b->release();
     delete T;
     d->tree = nullptr;
@@ -1256,7 +1498,7 @@ REB_API long reb_amd_tree_dump(struct reb_simulation* r, double* out, long cap) 
     using namespace rbamd;
     mark_host_newer(r);
     if (!ensure_device(r)) return -1;
-    if (!tree_build(r)) return -1;
+    if (!tree_build(r, TREE_GRAVITY)) return -1;
     return tree_dump_device(r, out, cap);
 }
 
