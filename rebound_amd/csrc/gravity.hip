@@ -406,6 +406,14 @@ __device__ __forceinline__ double vreg_const(double v) {
     return v;
 }
 
+// kahan_add of the product w d, unrounded: one operation less, one rounding less.
+__device__ __forceinline__ void kahan_fma(double w, double d, double& a, double& c) {
+    const double yv = fma(w, d, -c);
+    const double tv = a + yv;
+    c = (tv - a) - yv;
+    a = tv;
+}
+
 template <int MODE, bool CHECK>
 __device__ __forceinline__ void pair_tile(const double4* __restrict__ tile, int n,
                                           int jbase, int i, int ignore, double gx, double gy, double gz,
@@ -433,9 +441,9 @@ __device__ __forceinline__ void pair_tile(const double4* __restrict__ tile, int 
             if (skip_pair(i, j, ignore)) w = 0.;
         }
         if (MODE == FM_COMP) {
-            kahan_add(w * dx, sx, cx);
-            kahan_add(w * dy, sy, cy);
-            kahan_add(w * dz, sz, cz);
+            kahan_fma(w, dx, sx, cx);
+            kahan_fma(w, dy, sy, cy);
+            kahan_fma(w, dz, sz, cz);
         } else {
             sx = fma(w, dx, sx);
             sy = fma(w, dy, sy);
@@ -1006,14 +1014,14 @@ static std::vector<int2> sym_tasks(const SymPlan& p) {
     return t;
 }
 
-// Number of source chunks for the fast modes: enough workgroups to fill every
-// SIMD of the 256-CU part several times over, chunks no shorter than
-// kMinChunk sources (short chunks keep the time of one step small for N of a
-// few thousand, where a single workgroup's chunk sets the kernel's duration).
+// Number of source chunks for the fast modes: chunks no shorter than kMinChunk
+// sources (short chunks keep the time of one step small for N of a few
+// thousand, where a single workgroup's chunk sets the kernel's duration), and
+// at most max_chunks of them, which the workspaces are sized for.
 static constexpr int kMinChunk = 32;
 static_assert(kFast % kMinChunk == 0, "chunks tile the LDS tile");
 static int round_chunk(int c) { return ((c + kMinChunk - 1) / kMinChunk) * kMinChunk; }
-static int pick_chunks(int n_recv, int n_src, int ngb) {
+static int max_chunks(int n_recv, int n_src, int ngb) {
     const int blocks_x = (n_recv + kFast - 1) / kFast;
     const int target_blocks = 2048 * 256 / kFast;
     int s = (target_blocks + blocks_x - 1) / blocks_x;
@@ -1023,6 +1031,17 @@ static int pick_chunks(int n_recv, int n_src, int ngb) {
     if (s > 64) s = 64;
     if (s < 1) s = 1;
     return s;
+}
+// max_chunks rounds up, so that at many sizes a few workgroups more than the 2048
+// of two full rounds (four wavefronts on every SIMD) start a third: one chunk
+// fewer then (30011 targets, 20011 sources, FP64: 489 us with 118 x 18 workgroups, 469
+// with 118 x 17).  With half a workgroup per CU or more left over the third round
+// is worth its chunks (65000 targets, 20000 sources: 930 us with 254 x 9, 942 with 254
+// x 8).
+static int pick_chunks(int n_recv, int n_src, int ngb) {
+    const int s = max_chunks(n_recv, n_src, ngb);
+    const long blocks = (n_recv + kFast - 1) / kFast;
+    return s > 2 && blocks * s > 2048 && blocks * s <= 2048 + 128 ? s - 1 : s;
 }
 
 static size_t workspace_bytes(int n, int nchunk) { return sizeof(double) * 6 * (size_t)n * (size_t)nchunk; }
@@ -1604,7 +1623,7 @@ extern "C" {
 
 REB_API size_t reb_amd_gravity_workspace_bytes(size_t N, int precision) {
     if (precision == REB_AMD_PRECISION_EXACT) return 256;
-    return workspace_bytes((int)N, pick_chunks((int)N, (int)N, 1)) + 256;
+    return workspace_bytes((int)N, max_chunks((int)N, (int)N, 1)) + 256;
 }
 
 REB_API int reb_amd_gravity_direct(const double* x, const double* y, const double* z, const double* m, double* ax,
