@@ -32,8 +32,9 @@ FLOP_PER_PAIR = {"fp64": 20, "compensated": 28, "split": 28, "exact": 20}
 # reference's serial loop, gravity.c:195-214 (3 sub, 3 mul + 3 add for r^2
 # with softening, sqrt, 2 mul for r^3, div, 2 mul by the masses, 6 mul + 6 add
 # into both bodies) = 27; split precision 27 + 8 (the FP32 part counted apart
-# as in the one-sided kernel's 28 = 15 FP64 + 13 FP32 per ordered pair).
-FLOP_PER_SYM_PAIR = {"fp64": 27, "split": 35}
+# as in the one-sided kernel's 28 = 15 FP64 + 13 FP32 per ordered pair);
+# compensated 27 + 2 x 8 (the Kahan operations of the 28 per ordered pair).
+FLOP_PER_SYM_PAIR = {"fp64": 27, "split": 35, "compensated": 43}
 
 
 def profiled(what, kernel, workload_tag):
@@ -105,7 +106,7 @@ def run_mode(amd, args, name, precision, gravity, steps, warmup):
     sym = kp < pairs
     if sym:
         units, flop_unit, unit = kp / 2.0, FLOP_PER_SYM_PAIR[name], "unordered pair"
-        kernel = "k_direct_sym<%s>" % ("FM_SPLIT" if name == "split" else "FM_FP64")
+        kernel = "k_direct_sym<%s>" % {"fp64": "FM_FP64", "split": "FM_SPLIT", "compensated": "FM_COMP"}[name]
     else:
         units, flop_unit, unit = kp, FLOP_PER_PAIR[name], "ordered pair"
         kernel = "k_exact" if name == "exact" else "k_direct_fast<%s>" % (

@@ -724,14 +724,46 @@ __host__ __device__ __forceinline__ int sym_task(int A, int B, int nsb) {
     return A * nsb - A * (A + 1) / 2 + (B - A - 1);
 }
 
+// Sums of three components; COMPENSATED gravity carries their Kahan corrections.
+template <int MODE>
+struct Sum3 {
+    double x = 0., y = 0., z = 0.;
+    __device__ __forceinline__ void add(double w, double dx, double dy, double dz) {
+        x = fma(w, dx, x);
+        y = fma(w, dy, y);
+        z = fma(w, dz, z);
+    }
+    __device__ __forceinline__ void rotate() {
+        x = dpp_ror1(x);
+        y = dpp_ror1(y);
+        z = dpp_ror1(z);
+    }
+};
+template <>
+struct Sum3<FM_COMP> {
+    double x = 0., y = 0., z = 0., cx = 0., cy = 0., cz = 0.;
+    __device__ __forceinline__ void add(double w, double dx, double dy, double dz) {
+        kahan_fma(w, dx, x, cx);
+        kahan_fma(w, dy, y, cy);
+        kahan_fma(w, dz, z, cz);
+    }
+    __device__ __forceinline__ void rotate() {
+        x = dpp_ror1(x);
+        y = dpp_ror1(y);
+        z = dpp_ror1(z);
+        cx = dpp_ror1(cx);
+        cy = dpp_ror1(cy);
+        cz = dpp_ror1(cz);
+    }
+};
+
 // One J-block's 64 steps for the lane's targets.  CHECK: the J-block is the
 // last, ragged one of the bodies (its first jlim sources exist).
 template <int MODE, bool CHECK>
 __device__ __forceinline__ void sym_jblock(const double4* __restrict__ src, int k, int jlim, const double* tx,
                                            const double* ty, const double* tz, const double* tm, double soft2,
-                                           double c15, double c1875, double* bx, double* by, double* bz, double& jx,
-                                           double& jy, double& jz) {
-#pragma unroll 4
+                                           double c15, double c1875, Sum3<MODE>* b, Sum3<MODE>& j) {
+#pragma unroll MODE == FM_COMP ? 1 : 4
     for (int s = 0; s < kSymJB; s++) {
         const int idx = (k - s) & (kSymJB - 1);     // the source's index in the J-block
         const double4 sj = src[k + kSymJB - s];
@@ -749,18 +781,10 @@ __device__ __forceinline__ void sym_jblock(const double4* __restrict__ src, int 
                 wr = rinv3_fp64(r2, c15, c1875);
             }
             if (CHECK && idx >= jlim) wr = 0.;
-            const double wj = wr * sj.w;
-            const double wi = wr * tm[q];
-            bx[q] = fma(wj, dx, bx[q]);
-            by[q] = fma(wj, dy, by[q]);
-            bz[q] = fma(wj, dz, bz[q]);
-            jx = fma(wi, dx, jx);
-            jy = fma(wi, dy, jy);
-            jz = fma(wi, dz, jz);
+            b[q].add(wr * sj.w, dx, dy, dz);
+            j.add(wr * tm[q], dx, dy, dz);
         }
-        jx = dpp_ror1(jx);
-        jy = dpp_ror1(jy);
-        jz = dpp_ror1(jz);
+        j.rotate();
     }
 }
 
@@ -780,7 +804,9 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
     // J-block sources (x, y, z, m), double-buffered, each stored twice in a
     // row so that lane k reads entry k + 64 - s at step s without wrapping
     __shared__ double4 jt[2][2 * kSymJB];
-    __shared__ double jred[2][4][3][kSymJB];       // per-wave source sums of a J-block
+    constexpr bool COMP = MODE == FM_COMP;
+    constexpr int NC = COMP ? 6 : 3;               // values per body in the partials
+    __shared__ double jred[2][4][NC][kSymJB];      // per-wave source sums of a J-block
     const int tid = threadIdx.x;
     if ((int)blockIdx.x >= ntasks * split) {
         static_assert(sizeof(jt) >= sizeof(double4) * kFast, "the one-sided tile fits the J-block buffers");
@@ -798,7 +824,7 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
     const int w = tid >> 6, k = tid & 63;
     // targets of this lane (A < B: never the ragged superblock)
     double tx[kSymTPL], ty[kSymTPL], tz[kSymTPL], tm[kSymTPL];
-    double sx[kSymTPL], sy[kSymTPL], sz[kSymTPL];
+    Sum3<MODE> sum[kSymTPL];
 #pragma unroll
     for (int q = 0; q < kSymTPL; q++) {
         const int i = A * kSymSB + w * 64 * kSymTPL + q * 64 + k;
@@ -806,7 +832,6 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
         ty[q] = y[i];
         tz[q] = z[i];
         tm[q] = m[i];
-        sx[q] = sy[q] = sz[q] = 0.;
     }
     const int jbase = B * kSymSB;
     constexpr int NJB = kSymSB / kSymJB;
@@ -828,8 +853,20 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
     auto flush = [&](int jb) {
         if (w >= 3) return;
         const double* r = &jred[jb & 1][0][w][k];
-        const double v = ((r[0] + r[3 * kSymJB]) + r[6 * kSymJB]) + r[9 * kSymJB];
-        jpart[((size_t)t * 3 + w) * kSymSB + jb * kSymJB + k] = v;
+        constexpr int W = NC * kSymJB;             // from wave to wave
+        double* out = jpart + ((size_t)t * NC + w) * kSymSB + jb * kSymJB + k;
+        if constexpr (COMP) {
+            double v = r[0], c = r[3 * kSymJB];
+#pragma unroll
+            for (int q = 1; q < 4; q++) {
+                kahan_add(r[q * W], v, c);
+                kahan_add(-r[q * W + 3 * kSymJB], v, c);
+            }
+            out[0] = v;
+            out[3 * kSymSB] = c;
+        } else {
+            out[0] = ((r[0] + r[W]) + r[2 * W]) + r[3 * W];
+        }
     };
     const double c15 = vreg_const(1.5);
     const double c1875 = vreg_const(1.875);
@@ -841,35 +878,46 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
             jt[(jb + 1) & 1][tid + kSymJB] = nxt;
             nxt = source(jb + 2);
         }
-        double bx[kSymTPL], by[kSymTPL], bz[kSymTPL];
-#pragma unroll
-        for (int q = 0; q < kSymTPL; q++) bx[q] = by[q] = bz[q] = 0.;
-        double jx = 0., jy = 0., jz = 0.;
+        // FP64 and split: the J-block's sums apart, then added to the running ones
+        Sum3<MODE> part3[kSymTPL], src3;
+        Sum3<MODE>* b = COMP ? sum : part3;
         const int jlim = N - (jbase + jb * kSymJB);
         if (jlim >= kSymJB)
-            sym_jblock<MODE, false>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, bx, by, bz, jx, jy, jz);
+            sym_jblock<MODE, false>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, b, src3);
         else
-            sym_jblock<MODE, true>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, bx, by, bz, jx, jy, jz);
+            sym_jblock<MODE, true>(jt[jb & 1], k, jlim, tx, ty, tz, tm, soft2, c15, c1875, b, src3);
+        if constexpr (!COMP) {
 #pragma unroll
-        for (int q = 0; q < kSymTPL; q++) {
-            sx[q] += bx[q];
-            sy[q] += by[q];
-            sz[q] += bz[q];
+            for (int q = 0; q < kSymTPL; q++) {
+                sum[q].x += part3[q].x;
+                sum[q].y += part3[q].y;
+                sum[q].z += part3[q].z;
+            }
         }
         double* jr = &jred[jb & 1][w][0][k];
-        jr[0] = jx;
-        jr[kSymJB] = jy;
-        jr[2 * kSymJB] = jz;
+        jr[0] = src3.x;
+        jr[kSymJB] = src3.y;
+        jr[2 * kSymJB] = src3.z;
+        if constexpr (COMP) {
+            jr[3 * kSymJB] = src3.cx;
+            jr[4 * kSymJB] = src3.cy;
+            jr[5 * kSymJB] = src3.cz;
+        }
     }
     __syncthreads();
     if (jb1 > jb0) flush(jb1 - 1);
 #pragma unroll
     for (int q = 0; q < kSymTPL; q++) {
         const int li = w * 64 * kSymTPL + q * 64 + k;
-        double* p = ipart + ((size_t)t * split + part) * 3 * kSymSB + li;
-        p[0] = sx[q];
-        p[kSymSB] = sy[q];
-        p[2 * kSymSB] = sz[q];
+        double* p = ipart + ((size_t)t * split + part) * NC * kSymSB + li;
+        p[0] = sum[q].x;
+        p[kSymSB] = sum[q].y;
+        p[2 * kSymSB] = sum[q].z;
+        if constexpr (COMP) {
+            p[3 * kSymSB] = sum[q].cx;
+            p[4 * kSymSB] = sum[q].cy;
+            p[5 * kSymSB] = sum[q].cz;
+        }
     }
 }
 
@@ -878,7 +926,9 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
 // takes 64 bodies of one superblock; its four wavefronts each sum a quarter of
 // the partials (the loads of eight in flight), and the first adds the four
 // sums in order.  A body of superblock X has X source-side sums, kSymDiag one-sided
-// sums with their carries, and `split` target-side sums per later superblock.
+// sums with their carries, and `split` target-side sums per later superblock; CARRY: the
+// others come with carries too (COMPENSATED).
+template <bool CARRY>
 __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ ipart,
                                                     const double* __restrict__ jpart,
                                                     const double* __restrict__ dpart, int N, int nsb, int split,
@@ -891,24 +941,28 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
     const int X = first / kSymSB, loc = first % kSymSB;
     const int ii = min(i, N - 1) - first;          // lanes past the end read the last body's
     double s[3] = {0., 0., 0.}, c[3] = {0., 0., 0.};
-    const int total = X + 2 * kSymDiag + (nsb - 1 - X) * split;
+    constexpr int PER = CARRY ? 2 : 1;             // entries per partial sum: itself, its carry
+    const int total = PER * X + 2 * kSymDiag + PER * (nsb - 1 - X) * split;
     const int e0 = total * w / 4, e1 = total * (w + 1) / 4;
     // entry e: base pointer of its first component, component stride, sign
     auto load = [&](int e, double* v) {
         const double* p;
         size_t stride = kSymSB;
         double sign = 1.;
-        if (e < X) {
-            p = jpart + (size_t)sym_task(e, X, nsb) * 3 * kSymSB + loc;
-            sign = -1.;
-        } else if (e < X + 2 * kSymDiag) {
-            const int q = e - X;
+        if (e < PER * X) {
+            const int carry = e % PER;
+            p = jpart + ((size_t)sym_task(e / PER, X, nsb) * 3 * PER + 3 * carry) * kSymSB + loc;
+            sign = carry ? 1. : -1.;
+        } else if (e < PER * X + 2 * kSymDiag) {
+            const int q = e - PER * X;
             p = dpart + ((size_t)(q >> 1) * 6 + (q & 1 ? 3 : 0)) * N + first;
             stride = N;
             sign = q & 1 ? -1. : 1.;
         } else {
-            const int q = e - X - 2 * kSymDiag;
-            p = ipart + ((size_t)sym_task(X, X + 1 + q / split, nsb) * split + q % split) * 3 * kSymSB + loc;
+            const int q = (e - PER * X - 2 * kSymDiag) / PER, carry = (e - PER * X - 2 * kSymDiag) % PER;
+            const size_t part = (size_t)sym_task(X, X + 1 + q / split, nsb) * split + q % split;
+            p = ipart + (part * 3 * PER + 3 * carry) * kSymSB + loc;
+            sign = carry ? -1. : 1.;
         }
 #pragma unroll
         for (int f = 0; f < 3; f++) v[f] = sign * p[f * stride + ii];
@@ -990,12 +1044,12 @@ static int sym_split(int ntasks) {
     return best;
 }
 
-static SymPlan sym_plan(int N) {
+static SymPlan sym_plan(int N, bool compensated) {
     SymPlan p;
     p.nsb = (N + kSymSB - 1) / kSymSB;
     p.ntasks = p.nsb * (p.nsb - 1) / 2;
     p.split = sym_split(p.ntasks);
-    const size_t part = sizeof(double) * 3 * (size_t)kSymSB * (size_t)p.ntasks;
+    const size_t part = sizeof(double) * (compensated ? 6 : 3) * (size_t)kSymSB * (size_t)p.ntasks;
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.ipart_off = 0;
     p.jpart_off = up(part * p.split);
@@ -1073,10 +1127,14 @@ int seg_fast_mode(int precision, int compensated) {
 // Whether a simulation of N bodies, all active, without ghost boxes or
 // ignored terms, takes the symmetric path in this precision and gravity, and
 // the workspace it then needs.
-bool gravity_symmetric_path(size_t N, int precision, bool compensated) {
-    return !compensated && precision != REB_AMD_PRECISION_EXACT && N >= (size_t)kSymMinN;
+bool gravity_symmetric_path(size_t N, int precision) {
+    return precision != REB_AMD_PRECISION_EXACT && N >= (size_t)kSymMinN;
 }
-size_t gravity_symmetric_bytes(size_t N) { return sym_plan((int)N).bytes; }
+size_t gravity_symmetric_bytes(size_t N, bool compensated) { return sym_plan((int)N, compensated).bytes; }
+size_t gravity_symmetric_bytes_unsplit(size_t N) {
+    const size_t nsb = (N + kSymSB - 1) / kSymSB, tasks = nsb * (nsb - 1) / 2;
+    return tasks * (2 * 3 * sizeof(double) * kSymSB + sizeof(int2)) + 6 * sizeof(double) * N;
+}
 
 // Ordered pairs inside the superblocks (evaluated one-sided): sum over superblocks of n_A^2, self pairs included.
 static double sym_diag_pairs(int N) {
@@ -1095,15 +1153,15 @@ static int sym_launch(int mode, const double* x, const double* y, const double* 
     const int2* tasks = reinterpret_cast<const int2*>(base + plan.tasks_off);
     const dim3 grid(plan.ntasks * plan.split + (N + kFast - 1) / kFast * kSymDiag);
     if (ev) (void)hipEventRecord(ev[0], st);
-    if (mode == FM_SPLIT)
-        hipLaunchKernelGGL(k_direct_sym<FM_SPLIT>, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks,
-                           plan.split, soft2, tasks, ipart, jpart, dpart);
-    else
-        hipLaunchKernelGGL(k_direct_sym<FM_FP64>, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks,
-                           plan.split, soft2, tasks, ipart, jpart, dpart);
+    const auto pairs = mode == FM_COMP    ? k_direct_sym<FM_COMP>
+                       : mode == FM_SPLIT ? k_direct_sym<FM_SPLIT>
+                                          : k_direct_sym<FM_FP64>;
+    hipLaunchKernelGGL(pairs, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks, plan.split, soft2, tasks,
+                       ipart, jpart, dpart);
     if (ev) (void)hipEventRecord(ev[1], st);
-    hipLaunchKernelGGL(k_sym_reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb,
-                       plan.split, -G, ax, ay, az, kd);
+    const auto reduce = mode == FM_COMP ? k_sym_reduce<true> : k_sym_reduce<false>;
+    hipLaunchKernelGGL(reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb, plan.split, -G,
+                       ax, ay, az, kd);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -1289,8 +1347,8 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
     // Every body active, no ghost boxes, nothing ignored: each pair once
     // (Newton's third law); otherwise the one-sided kernels.
     if (ngb == 1 && N_active == N && r->gravity_ignore_terms == 0 &&
-        gravity_symmetric_path((size_t)N, d->precision, compensated)) {
-        const SymPlan plan = sym_plan(N);
+        gravity_symmetric_path((size_t)N, d->precision)) {
+        const SymPlan plan = sym_plan(N, compensated);
         if (!d->partial.ensure(plan.bytes)) {
             reb_simulation_error(r, "Out of device memory for the gravity workspace.");
             return false;
@@ -1306,7 +1364,7 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
             d->sym_tasks_dev = tasks;
         }
         if (d->profiling) d->kpairs += (double)N * (double)N - sym_diag_pairs(N);
-        const int mode = d->precision == REB_AMD_PRECISION_SPLIT ? FM_SPLIT : FM_FP64;
+        const int mode = seg_fast_mode(d->precision, compensated);
         const int rc = sym_launch(mode, d->field(FX), d->field(FY), d->field(FZ), d->field(FM), d->field(FAX),
                                   d->field(FAY), d->field(FAZ), N, r->G, soft2, plan, base, d->stream, ev, kd);
         if (rc) return RB_HIP(r, hipGetLastError());

@@ -164,8 +164,11 @@ std::vector<struct reb_vec6d> ghostboxes(struct reb_simulation* r, int nx, int n
 bool gravity_direct(struct reb_simulation* r, bool compensated, const double* kick_drift = nullptr);
 // The pair-symmetric direct-gravity path (gravity.hip) for N bodies, all
 // active, no ghost boxes, nothing ignored; its workspace in bytes.
-bool gravity_symmetric_path(size_t N, int precision, bool compensated);
-size_t gravity_symmetric_bytes(size_t N);
+bool gravity_symmetric_path(size_t N, int precision);
+size_t gravity_symmetric_bytes(size_t N, bool compensated);
+// What that workspace comes to without splitting tasks over workgroups or
+// carries: the least a job is charged for it.
+size_t gravity_symmetric_bytes_unsplit(size_t N);
 
 // Batched order-2 leapfrog steps with direct gravity for many independent
 // simulations (gravity.hip k_seg_*).  A SegJob holds one simulation's device

@@ -202,12 +202,20 @@ static double since(const Server* S) {
 
 static size_t whfast_footprint(size_t n) { return n * 17 * sizeof(double) + sizeof(WHSys) + 64; }
 
-static size_t nbody_footprint(size_t n, int precision, int gravity) {
+// least: with the force's smallest workspace, which decides whether a budget can
+// hold the job at all.  The larger workspaces of the fast paths are charged up to
+// the budget: a job that fits alone without them is not refused for them.
+static size_t nbody_footprint(size_t n, int precision, int gravity, bool least = false) {
     size_t cap = 64;
     while (cap < n) cap *= 2;
     size_t ws = reb_amd_gravity_workspace_bytes(n, precision);
-    if (gravity_symmetric_path(n, precision, gravity == REB_GRAVITY_COMPENSATED))
-        ws = std::max(ws, gravity_symmetric_bytes(n));
+    const bool compensated = gravity == REB_GRAVITY_COMPENSATED;
+    if (gravity_symmetric_path(n, precision)) {
+        if (!least)
+            ws = std::max(ws, gravity_symmetric_bytes(n, compensated));
+        else if (!compensated)
+            ws = std::max(ws, gravity_symmetric_bytes_unsplit(n));
+    }
     return NFIELD * cap * sizeof(double) + ws + 16 * n + 4096;
 }
 
@@ -216,7 +224,7 @@ static size_t nbody_footprint(size_t n, int precision, int gravity) {
 // kernels are one-sided, so a job's bits would otherwise depend on the route).
 static bool nbody_single(const Job* j) {
     return j->precision == REB_AMD_PRECISION_EXACT ||
-           gravity_symmetric_path(j->bodies.size(), j->precision, j->gravity == REB_GRAVITY_COMPENSATED);
+           gravity_symmetric_path(j->bodies.size(), j->precision);
 }
 
 // ------------------------------------------------------------------ pool memory
@@ -1167,6 +1175,9 @@ REB_API void reb_amd_server_free(struct reb_amd_server* h) {
 
 static long submit(Server* S, std::unique_ptr<Job> j) {
     std::lock_guard<std::mutex> g(S->mu);
+    if (j->kind == JOB_NBODY && j->footprint > S->budget &&
+        nbody_footprint(j->bodies.size(), j->precision, j->gravity, true) <= S->budget)
+        j->footprint = S->budget;
     if (j->footprint > S->budget) {
         S->err = "job footprint (" + std::to_string(j->footprint) + " bytes) exceeds the memory budget";
         set_last_error(S->err);
