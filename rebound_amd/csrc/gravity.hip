@@ -24,7 +24,9 @@
 #include <cmath>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
+#include "ieee_mid.h"
 #include "internal.h"
 
 namespace rbamd {
@@ -54,6 +56,20 @@ static constexpr int kMaxGB = 125;       // N_ghost up to 2 in all three axes
 struct GBList {
     int n;
     GB3 g[kMaxGB];
+    bool zero() const { return n == 1 && g[0].x == 0. && g[0].y == 0. && g[0].z == 0.; }
+};
+
+// Ghost-box offsets of a pass: the list of the simulation (kernel argument) or
+// the single zero offset of a simulation without ghost boxes, whose kernels then
+// carry no 3 KB list in their arguments and wait for no read of it.
+struct GBFromList {
+    GBList gl;
+    __device__ int n() const { return gl.n; }
+    __device__ const GB3& get(int g) const { return gl.g[g]; }
+};
+struct GBZero {
+    __device__ int n() const { return 1; }
+    __device__ GB3 get(int) const { return GB3{0., 0., 0.}; }
 };
 
 // The leapfrog's kick and closing drift, applied by the pass that finishes the
@@ -84,135 +100,185 @@ __device__ __forceinline__ void kahan_add(double term, double& a, double& c) {
 // targets), :346-378 (test-particle targets), :379-410 (active targets feel
 // test particles), no ghost boxes, Kahan sums.
 //
-// The terms are independent: all 256 threads of a workgroup compute them for
-// TGT targets x TILE sources at a time (IEEE sqrt and division, no
-// contraction: the reference's expressions) into LDS rows, one row per
-// (target, component), and one lane per row then adds its row in ascending
-// source order: the reference's sequential sum, each component its own
-// chain.  The rows are double-buffered, so one barrier per tile suffices and
-// the summing lanes' chains overlap the other waves' terms of the next tile;
-// each thread loads its sources one tile ahead.
-static constexpr int kExThreads = 256;
-static constexpr int kExactRowwiseN = 49152;   // from here on the row-wise kernels
+// The terms are independent: four wavefronts of a workgroup compute them for
+// TGT targets x TILE sources at a time (the reference's expressions, no
+// contraction) into LDS rows, one row per (target, component), and a fifth
+// wavefront adds the previous tile's rows meanwhile, one lane per row, in
+// ascending source order: the reference's sequential sum, each component its own
+// chain.  The rows are double-buffered, so one barrier per tile suffices.  Small N
+// is bound by the chains (N dependent additions), so the summing lanes read their row
+// sixteen terms ahead.  1024 bodies 27 -> 17 us with the terms and the sums on
+// separate wavefronts and these reads; staging the sources in LDS four tiles ahead
+// gained nothing there and lost 15 % from 8192 bodies (fewer workgroups per CU).
+static constexpr int kExTermThreads = 256;
+static constexpr int kExThreads = kExTermThreads + 64;
 
-template <bool COMP, int TGT, int TILE>
+// PER pair factors of one target: -G / r^3 (BASIC, gravity.c:222-230) or
+// G / (r^2 r) (COMPENSATED, :315-341), from the short IEEE sequences of
+// ieee_mid.h while every operand is in their range.
+template <bool COMP, int PER>
+__device__ __forceinline__ void exact_factors(const double* r2, double G, bool g_mid, double* f) {
+    unsigned int far = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        far = max(far, mid_distance(r2[q]));
+        const double r = sqrt_mid(r2[q]);
+        f[q] = COMP ? div_mid(G, r2[q] * r) : div_mid(-G, r * r * r);
+    }
+    if (!g_mid || far >= kMidSpan) {
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const double r = sqrt(r2[q]);
+            f[q] = COMP ? G / (r2[q] * r) : -G / (r * r * r);
+        }
+    }
+}
+
+template <bool COMP, int TGT, int TILE, class GBS>
 __global__ __launch_bounds__(kExThreads) void k_exact(const double* __restrict__ x, const double* __restrict__ y,
                                                        const double* __restrict__ z, const double* __restrict__ m,
                                                        double* __restrict__ ax, double* __restrict__ ay,
                                                        double* __restrict__ az, int N, int N_active, int tp_type,
-                                                       int ignore, double G, double soft2, GBList gl) {
-    constexpr int PER = TGT * TILE / kExThreads;   // terms per thread and tile
+                                                       int ignore, double G, double soft2, GBS gbs) {
+    constexpr int PER = TGT * TILE / kExTermThreads;   // terms per thread and tile
     constexpr int ROWS = 3 * TGT;
-    constexpr int PITCH = TILE + 2;                // row pitch (doubles): 16-byte aligned rows, spread banks
-    static_assert(PER >= 1 && PER * kExThreads == TGT * TILE, "tile shape");
-    static_assert(ROWS <= kExThreads, "one summing lane per row");
+    constexpr int PITCH = TILE + 2;                    // row pitch (doubles): 16-byte aligned rows, spread banks
+    static_assert(PER % 2 == 0 && PER * kExTermThreads == TGT * TILE && kExTermThreads % TGT == 0, "tile shape");
+    static_assert(ROWS <= 64 && TILE % 32 == 0, "one summing lane per row, rows read in sixteens");
     __shared__ __align__(16) double T[2][ROWS][PITCH];
     const int tid = threadIdx.x;
     const int i0 = blockIdx.x * TGT;
-    // term phase: thread -> (target ti, sources tj0 .. tj0 + PER - 1 of a tile)
-    const int ti = tid % TGT;
-    const int tj0 = (tid / TGT) * PER;
-    const int i = i0 + ti;
-    const bool live = i < N;
-    const double xi = live ? x[i] : 0., yi = live ? y[i] : 0., zi = live ? z[i] : 0.;
-    // sum phase: lanes 0 .. ROWS-1, lane -> (target si, component sc)
-    const int si = i0 + tid / 3;
-    const int sc = tid % 3;
-    const bool summer = tid < ROWS && si < N;
-    double acc = 0., comp = 0.;
+    const int ngb = gbs.n();
     int buf = 0;
-    const int ngb = COMP ? 1 : gl.n;
+    if (tid < kExTermThreads) {
+        // thread -> (target ti, sources tj0 .. tj0 + PER - 1 of a tile)
+        const int ti = tid % TGT;
+        const int tj0 = (tid / TGT) * PER;
+        const int i = min(i0 + ti, N - 1);             // rows past the last target are not added
+        const double xi = x[i], yi = y[i], zi = z[i];
+        const bool g_mid = mid_distance(fabs(G)) < kMidSpan;
+        for (int g = 0; g < ngb; g++) {
+            const GB3 gb = gbs.get(g);
+            for (int pass = 0; pass < (tp_type ? 2 : 1); pass++) {
+                const int j0 = pass == 0 ? 0 : N_active;
+                const int j1 = pass == 0 ? N_active : N;
+                // this thread's sources, loaded two tiles ahead (a tile of small N
+                // takes 0.3 us, less than a fetch of what the drift just wrote)
+                double4 ahead[2][PER];
+                auto fetch = [&](int t, double4* o) {
+#pragma unroll
+                    for (int q = 0; q < PER; q++) {
+                        const int j = min(t + tj0 + q, j1 - 1);
+                        o[q] = make_double4(x[j], y[j], z[j], m[j]);
+                    }
+                };
+                auto tile = [&](int t, double4* o) {
+                    double dx[PER], dy[PER], dz[PER], r2[PER], f[PER], cm[PER];
+#pragma unroll
+                    for (int q = 0; q < PER; q++) {
+                        if (COMP) {
+                            dx[q] = xi - o[q].x;
+                            dy[q] = yi - o[q].y;
+                            dz[q] = zi - o[q].z;
+                        } else {
+                            dx[q] = (gb.x + xi) - o[q].x;
+                            dy[q] = (gb.y + yi) - o[q].y;
+                            dz[q] = (gb.z + zi) - o[q].z;
+                        }
+                        r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q] + soft2;
+                        cm[q] = o[q].w;
+                    }
+                    if (t + 2 * TILE < j1) fetch(t + 2 * TILE, o);
+                    exact_factors<COMP, PER>(r2, G, g_mid, f);
+#pragma unroll
+                    for (int q = 0; q < PER; q += 2) {
+                        const double w0 = (COMP ? -f[q] : f[q]) * cm[q];
+                        const double w1 = (COMP ? -f[q + 1] : f[q + 1]) * cm[q + 1];
+                        double2* row = reinterpret_cast<double2*>(&T[buf][3 * ti][tj0 + q]);
+                        row[0] = make_double2(w0 * dx[q], w1 * dx[q + 1]);
+                        row[PITCH / 2] = make_double2(w0 * dy[q], w1 * dy[q + 1]);
+                        row[PITCH] = make_double2(w0 * dz[q], w1 * dz[q + 1]);
+                    }
+                    // After this barrier the summers read T[buf]; the next writes
+                    // to T[buf] come two tiles later, after the next barrier,
+                    // which the summers reach only once this sum is done.
+                    __syncthreads();
+                    buf ^= 1;
+                };
+                if (j0 < j1) fetch(j0, ahead[0]);
+                if (j0 + TILE < j1) fetch(j0 + TILE, ahead[1]);
+                for (int t = j0; t < j1; t += 2 * TILE) {
+                    tile(t, ahead[0]);
+                    if (t + TILE < j1) tile(t + TILE, ahead[1]);
+                }
+            }
+        }
+        return;
+    }
+    // lanes 0 .. ROWS-1: (target si, component sc)
+    const int lane = tid - kExTermThreads;
+    const int si = i0 + lane / 3;
+    const int sc = lane % 3;
+    const bool summer = lane < ROWS && si < N;
+    double acc = 0., comp = 0.;
+    auto add = [&](double term) {
+        if (COMP)
+            kahan_add(term, acc, comp);
+        else
+            acc += term;
+    };
     for (int g = 0; g < ngb; g++) {
-        const GB3 gb = COMP ? GB3{0., 0., 0.} : gl.g[g];
-        for (int pass = 0; pass < 2; pass++) {
+        for (int pass = 0; pass < (tp_type ? 2 : 1); pass++) {
             const int j0 = pass == 0 ? 0 : N_active;
             const int j1 = pass == 0 ? N_active : N;
-            if (pass == 1 && !tp_type) break;
             // the second pass only reaches active targets
-            const bool tgt = live && !(pass == 1 && i >= N_active);
-            const bool stgt = summer && !(pass == 1 && si >= N_active);
-            auto skipped = [&](int ii, int j) {
-                if (COMP || pass == 0) return skip_pair(ii, j, ignore);
-                return (ignore == 1 && j == 1 && ii == 0) || (ignore == 2 && (j == 0 || ii == 0));
+            const bool mine = summer && !(pass == 1 && si >= N_active);
+            auto skipped = [&](int j) {
+                if (COMP || pass == 0) return skip_pair(si, j, ignore);
+                return (ignore == 1 && j == 1 && si == 0) || (ignore == 2 && (j == 0 || si == 0));
             };
-            // this thread's sources of the next tile, loaded one tile ahead
-            double nx[PER], ny[PER], nz[PER], nm[PER];
-            auto fetch = [&](int t) {
-#pragma unroll
-                for (int q = 0; q < PER; q++) {
-                    const int j = t + tj0 + q;
-                    if (j < j1) {
-                        nx[q] = x[j]; ny[q] = y[j]; nz[q] = z[j]; nm[q] = m[j];
-                    }
-                }
-            };
-            if (j0 < j1) fetch(j0);
             for (int t = j0; t < j1; t += TILE, buf ^= 1) {
                 const int n = min(TILE, j1 - t);
-                double cx[PER], cy[PER], cz[PER], cm[PER];
-#pragma unroll
-                for (int q = 0; q < PER; q++) {
-                    cx[q] = nx[q]; cy[q] = ny[q]; cz[q] = nz[q]; cm[q] = nm[q];
-                }
-                if (t + TILE < j1) fetch(t + TILE);
-#pragma unroll
-                for (int q = 0; q < PER; q++) {
-                    const int k = tj0 + q;
-                    const int j = t + k;
-                    if (!tgt || k >= n || skipped(i, j)) continue;
-                    double tx, ty, tz;
-                    if (COMP) {
-                        const double dx = xi - cx[q];
-                        const double dy = yi - cy[q];
-                        const double dz = zi - cz[q];
-                        const double r2 = dx * dx + dy * dy + dz * dz + soft2;
-                        const double rr = sqrt(r2);
-                        const double prefact = G / (r2 * rr);
-                        const double prefactj = -prefact * cm[q];
-                        tx = prefactj * dx;
-                        ty = prefactj * dy;
-                        tz = prefactj * dz;
-                    } else {
-                        const double dx = (gb.x + xi) - cx[q];
-                        const double dy = (gb.y + yi) - cy[q];
-                        const double dz = (gb.z + zi) - cz[q];
-                        const double _r = sqrt(dx * dx + dy * dy + dz * dz + soft2);
-                        const double prefact = -G / (_r * _r * _r) * cm[q];
-                        tx = prefact * dx;
-                        ty = prefact * dy;
-                        tz = prefact * dz;
-                    }
-                    T[buf][3 * ti + 0][k] = tx;
-                    T[buf][3 * ti + 1][k] = ty;
-                    T[buf][3 * ti + 2][k] = tz;
-                }
-                // After this barrier the summers read T[buf]; the next writes
-                // to T[buf] come two tiles later, after the next barrier, which
-                // the summers reach only once this sum is done.
                 __syncthreads();
-                if (stgt) {
-                    const double* row = T[buf][tid];
-                    auto add = [&](double term) {
-                        if (COMP) {
-                            const double yv = term - comp;
-                            const double tv = acc + yv;
-                            comp = (tv - acc) - yv;
-                            acc = tv;
-                        } else {
-                            acc += term;
+                if (!mine) continue;
+                const double2* row = reinterpret_cast<const double2*>(T[buf][lane]);
+                // Pairs the reference leaves out: the target itself and,
+                // with ignored terms, pairs with bodies 0 and 1.
+                const bool self = (COMP || pass == 0) && t <= si && si < t + n;
+                const bool rare = ignore != 0 && (t < 2 || si < 2);
+                const bool whole = !self && !rare && n == TILE;
+                double2 v[2][8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[0][k] = row[k];
+#pragma unroll
+                for (int h = 0; h < TILE / 16; h++) {
+                    if (h + 1 < TILE / 16) {
+#pragma unroll
+                        for (int k = 0; k < 8; k++) v[(h + 1) & 1][k] = row[8 * (h + 1) + k];
+                    }
+                    if (whole) {
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            add(v[h & 1][k].x);
+                            add(v[h & 1][k].y);
                         }
-                    };
-                    // Pairs the reference leaves out: the target itself and,
-                    // with ignored terms, pairs with bodies 0 and 1.
-                    const bool check = (t <= si && si < t + n) || (ignore != 0 && (t < 2 || si < 2));
-                    if (check) {
-                        for (int k = 0; k < n; k++)
-                            if (!skipped(si, t + k)) add(row[k]);
-                    } else if (n == TILE) {
-#pragma unroll 16
-                        for (int k = 0; k < TILE; k++) add(row[k]);
-                    } else {
-                        for (int k = 0; k < n; k++) add(row[k]);
+                        continue;
+                    }
+#pragma unroll
+                    for (int k = 0; k < 16; k++) {
+                        const int at = 16 * h + k;
+                        bool left_out = at >= n || (self && t + at == si);
+                        if (rare) left_out = left_out || skipped(t + at);
+                        const double term = k & 1 ? v[h & 1][k / 2].y : v[h & 1][k / 2].x;
+                        if (COMP) {
+                            const double s0 = acc, c0 = comp;
+                            add(term);
+                            acc = left_out ? s0 : acc;
+                            comp = left_out ? c0 : comp;
+                        } else {
+                            // a zero changes nothing: the sum starts from +0 and is never -0
+                            add(left_out ? 0. : term);
+                        }
                     }
                 }
             }
@@ -243,6 +309,7 @@ __global__ __launch_bounds__(kBlock) void k_basic_exact(
     const int blk_lo = blockIdx.x * kBlock, blk_hi = blk_lo + kBlock;
     const double xi = live ? x[i] : 0., yi = live ? y[i] : 0., zi = live ? z[i] : 0.;
     double a_x = 0., a_y = 0., a_z = 0.;
+    const bool g_mid = mid_distance(fabs(G)) < kMidSpan;
     for (int g = 0; g < gl.n; g++) {
         const GB3 gb = gl.g[g];
         for (int pass = 0; pass < 2; pass++) {
@@ -256,16 +323,27 @@ __global__ __launch_bounds__(kBlock) void k_basic_exact(
                 __syncthreads();
                 const int n = min(kBlock, j1 - t);
                 if (!live || (pass == 1 && i >= N_active)) continue;
-                auto term = [&](const double4 s) {
-                    const double dx = (gb.x + xi) - s.x;
-                    const double dy = (gb.y + yi) - s.y;
-                    const double dz = (gb.z + zi) - s.z;
-                    const double _r = sqrt(dx * dx + dy * dy + dz * dz + soft2);
-                    const double prefact = -G / (_r * _r * _r) * s.w;
-                    a_x += prefact * dx;
-                    a_y += prefact * dy;
-                    a_z += prefact * dz;
+                auto terms = [&](auto count, const double4* s) {
+                    constexpr int PER = decltype(count)::value;
+                    double dx[PER], dy[PER], dz[PER], r2[PER], f[PER];
+#pragma unroll
+                    for (int q = 0; q < PER; q++) {
+                        dx[q] = (gb.x + xi) - s[q].x;
+                        dy[q] = (gb.y + yi) - s[q].y;
+                        dz[q] = (gb.z + zi) - s[q].z;
+                        r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q] + soft2;
+                    }
+                    exact_factors<false, PER>(r2, G, g_mid, f);
+#pragma unroll
+                    for (int q = 0; q < PER; q++) {
+                        const double prefact = f[q] * s[q].w;
+                        a_x += prefact * dx[q];
+                        a_y += prefact * dy[q];
+                        a_z += prefact * dz[q];
+                    }
                 };
+                using One = std::integral_constant<int, 1>;
+                using Four = std::integral_constant<int, 4>;
                 // Tiles without this block's targets (and, with ignored terms,
                 // without bodies 0 and 1 as sources or among the block's
                 // targets) need no per-pair test: the terms are then
@@ -274,8 +352,9 @@ __global__ __launch_bounds__(kBlock) void k_basic_exact(
                 const bool check =
                     (pass == 0 && t < blk_hi && t + n > blk_lo) || (ignore != 0 && (t < 2 || blk_lo < 2));
                 if (!check) {
-#pragma unroll 4
-                    for (int k = 0; k < n; k++) term(tile[k]);
+                    int k = 0;
+                    for (; k + 4 <= n; k += 4) terms(Four{}, tile + k);
+                    for (; k < n; k++) terms(One{}, tile + k);
                     continue;
                 }
                 for (int k = 0; k < n; k++) {
@@ -286,7 +365,7 @@ __global__ __launch_bounds__(kBlock) void k_basic_exact(
                         if (ignore == 1 && j == 1 && i == 0) continue;
                         if (ignore == 2 && (j == 0 || i == 0)) continue;
                     }
-                    term(tile[k]);
+                    terms(One{}, tile + k);
                 }
             }
         }
@@ -312,6 +391,7 @@ __global__ __launch_bounds__(kBlock) void k_comp_exact(
     const int blk_lo = blockIdx.x * kBlock, blk_hi = blk_lo + kBlock;
     const double xi = live ? x[i] : 0., yi = live ? y[i] : 0., zi = live ? z[i] : 0.;
     double a_x = 0., a_y = 0., a_z = 0., c_x = 0., c_y = 0., c_z = 0.;
+    const bool g_mid = mid_distance(fabs(G)) < kMidSpan;
     for (int pass = 0; pass < 2; pass++) {
         int j0 = pass == 0 ? 0 : N_active;
         int j1 = pass == 0 ? N_active : N;
@@ -323,28 +403,38 @@ __global__ __launch_bounds__(kBlock) void k_comp_exact(
             __syncthreads();
             const int n = min(kBlock, j1 - t);
             if (!live || (pass == 1 && i >= N_active)) continue;
-            auto term = [&](const double4 s) {
-                const double dx = xi - s.x;
-                const double dy = yi - s.y;
-                const double dz = zi - s.z;
-                const double r2 = dx * dx + dy * dy + dz * dz + soft2;
-                const double rr = sqrt(r2);
-                const double prefact = G / (r2 * rr);
-                const double prefactj = -prefact * s.w;
-                kahan_add(prefactj * dx, a_x, c_x);
-                kahan_add(prefactj * dy, a_y, c_y);
-                kahan_add(prefactj * dz, a_z, c_z);
+            auto terms = [&](auto count, const double4* s) {
+                constexpr int PER = decltype(count)::value;
+                double dx[PER], dy[PER], dz[PER], r2[PER], f[PER];
+#pragma unroll
+                for (int q = 0; q < PER; q++) {
+                    dx[q] = xi - s[q].x;
+                    dy[q] = yi - s[q].y;
+                    dz[q] = zi - s[q].z;
+                    r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q] + soft2;
+                }
+                exact_factors<true, PER>(r2, G, g_mid, f);
+#pragma unroll
+                for (int q = 0; q < PER; q++) {
+                    const double prefactj = -f[q] * s[q].w;
+                    kahan_add(prefactj * dx[q], a_x, c_x);
+                    kahan_add(prefactj * dy[q], a_y, c_y);
+                    kahan_add(prefactj * dz[q], a_z, c_z);
+                }
             };
+            using One = std::integral_constant<int, 1>;
+            using Four = std::integral_constant<int, 4>;
             const bool check = (t < blk_hi && t + n > blk_lo) || (ignore != 0 && (t < 2 || blk_lo < 2));
             if (!check) {
-#pragma unroll 4
-                for (int k = 0; k < n; k++) term(tile[k]);
+                int k = 0;
+                for (; k + 4 <= n; k += 4) terms(Four{}, tile + k);
+                for (; k < n; k++) terms(One{}, tile + k);
                 continue;
             }
             for (int k = 0; k < n; k++) {
                 const int j = t + k;
                 if (skip_pair(i, j, ignore)) continue;
-                term(tile[k]);
+                terms(One{}, tile + k);
             }
         }
     }
@@ -355,16 +445,19 @@ __global__ __launch_bounds__(kBlock) void k_comp_exact(
     }
 }
 
+// Measured on gfx950 (leapfrog steps; the start of the lines: sums and terms on the
+// same wavefront, sources one tile ahead, full-range square root and division):
+// 8 targets x 64 sources beat 16 x 64 at every N (1024 bodies 23.5 us against 29.9,
+// 16384 0.70 ms against 0.99; before 32.0 and 0.86), and the row-wise kernel from
+// about 57000 (49152 bodies 5.7 ms against 6.4, 65536 9.9 against 8.5; before 6.6
+// and 8.9).
+static constexpr int kExactRowwiseN = 57344;
+
 template <bool COMP>
 static void launch_exact(hipStream_t st, const double* x, const double* y, const double* z, const double* m,
                          double* ax, double* ay, double* az, int N, int N_active, int tp_type, int ignore, double G,
                          double soft2, const GBList& gl) {
-    // Measured on gfx950 (shapes 16x16 .. 1x256 targets x sources, N = 256
-    // .. 65536): 8 targets x 64 sources is within 10 % of the best shape at
-    // every N below ~50k; the row-wise kernel wins above.
-#define RB_EXACT(TGT, TILE)                                                                                           \
-    hipLaunchKernelGGL((k_exact<COMP, TGT, TILE>), dim3((N + TGT - 1) / TGT), dim3(kExThreads), 0, st, x, y, z, m,   \
-                       ax, ay, az, N, N_active, tp_type, ignore, G, soft2, gl)
+    const dim3 grid((N + 7) / 8);
     if (N >= kExactRowwiseN) {
         if (COMP)
             hipLaunchKernelGGL(k_comp_exact, dim3((N + kBlock - 1) / kBlock), dim3(kBlock), 0, st, x, y, z, m, ax,
@@ -372,10 +465,13 @@ static void launch_exact(hipStream_t st, const double* x, const double* y, const
         else
             hipLaunchKernelGGL(k_basic_exact, dim3((N + kBlock - 1) / kBlock), dim3(kBlock), 0, st, x, y, z, m, ax,
                                ay, az, N, N_active, tp_type, ignore, G, soft2, gl);
+    } else if (COMP || gl.zero()) {
+        hipLaunchKernelGGL((k_exact<COMP, 8, 64, GBZero>), grid, dim3(kExThreads), 0, st, x, y, z, m, ax, ay, az, N,
+                           N_active, tp_type, ignore, G, soft2, GBZero{});
     } else {
-        RB_EXACT(8, 64);
+        hipLaunchKernelGGL((k_exact<false, 8, 64, GBFromList>), grid, dim3(kExThreads), 0, st, x, y, z, m, ax, ay,
+                           az, N, N_active, tp_type, ignore, G, soft2, GBFromList{gl});
     }
-#undef RB_EXACT
 }
 
 // ---------------------------------------------------------------- FP64 / SPLIT / COMP-FP64
@@ -452,18 +548,6 @@ __device__ __forceinline__ void pair_tile(const double4* __restrict__ tile, int 
     }
 }
 
-// Ghost-box offsets of a pass: the list of the simulation (kernel argument) or
-// the single zero offset of a simulation without ghost boxes.
-struct GBFromList {
-    const GBList& gl;
-    __device__ int n() const { return gl.n; }
-    __device__ GB3 get(int g) const { return gl.g[g]; }
-};
-struct GBZero {
-    __device__ int n() const { return 1; }
-    __device__ GB3 get(int) const { return GB3{0., 0., 0.}; }
-};
-
 // One workgroup of the pair kernel: targets bx*kFast.. of n_recv, sources of
 // chunk `by` of [j_begin, j_end).  Writes the chunk's sums and carries to
 // `partial` (pstride doubles per component).
@@ -535,14 +619,14 @@ __device__ __forceinline__ void direct_fast_block(const double* __restrict__ x, 
 // Four wavefronts per SIMD (128 VGPRs, no spills in the pair loop) measured
 // faster than eight on gfx950; at N=65536 the grid is 256 target blocks x 8
 // source chunks.
-template <int MODE>
+template <int MODE, class GBS>
 __global__ __launch_bounds__(kFast) __attribute__((amdgpu_waves_per_eu(RB_FAST_WAVES, RB_FAST_WAVES))) void k_direct_fast(
     const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
     const double* __restrict__ m, int n_recv, int j_begin, int j_end, int chunk, int ignore, double soft2,
-    GBList gl, double* __restrict__ partial, int pstride) {
+    GBS gbs, double* __restrict__ partial, int pstride) {
     __shared__ double4 tile[kFast];
-    direct_fast_block<MODE>(x, y, z, m, n_recv, j_begin, j_end, chunk, ignore, soft2, GBFromList{gl}, partial,
-                            pstride, (int)blockIdx.x, (int)blockIdx.y, tile);
+    direct_fast_block<MODE>(x, y, z, m, n_recv, j_begin, j_end, chunk, ignore, soft2, gbs, partial, pstride,
+                            (int)blockIdx.x, (int)blockIdx.y, tile);
 }
 
 // Sum the chunk partials in chunk order (Kahan), apply -G and write (or add to)
@@ -1175,20 +1259,18 @@ static int launch_fast(int mode, const double* x, const double* y, const double*
     const int used = nsrc > 0 ? (nsrc + chunk - 1) / chunk : 1;
     dim3 grid((n_recv + kFast - 1) / kFast, used);
     if (ev) (void)hipEventRecord(ev[0], st);
-    switch (mode) {
-        case FM_FP64:
-            hipLaunchKernelGGL(k_direct_fast<FM_FP64>, grid, dim3(kFast), 0, st, x, y, z, m, n_recv, j_begin, j_end,
-                               chunk, ignore, soft2, gl, partial, n_recv);
-            break;
-        case FM_SPLIT:
-            hipLaunchKernelGGL(k_direct_fast<FM_SPLIT>, grid, dim3(kFast), 0, st, x, y, z, m, n_recv, j_begin,
-                               j_end, chunk, ignore, soft2, gl, partial, n_recv);
-            break;
-        default:
-            hipLaunchKernelGGL(k_direct_fast<FM_COMP>, grid, dim3(kFast), 0, st, x, y, z, m, n_recv, j_begin, j_end,
-                               chunk, ignore, soft2, gl, partial, n_recv);
-            break;
-    }
+    auto pairs = [&](auto gbs) {
+        using GBS = decltype(gbs);
+        const auto k = mode == FM_FP64    ? k_direct_fast<FM_FP64, GBS>
+                       : mode == FM_SPLIT ? k_direct_fast<FM_SPLIT, GBS>
+                                          : k_direct_fast<FM_COMP, GBS>;
+        hipLaunchKernelGGL(k, grid, dim3(kFast), 0, st, x, y, z, m, n_recv, j_begin, j_end, chunk, ignore, soft2, gbs,
+                           partial, n_recv);
+    };
+    if (gl.zero())
+        pairs(GBZero{});
+    else
+        pairs(GBFromList{gl});
     if (ev) (void)hipEventRecord(ev[1], st);
     hipLaunchKernelGGL(k_reduce, dim3((n_recv + 255) / 256), dim3(256), 0, st, partial, n_recv, used, n_recv, -G,
                        accumulate, ignore, ax, ay, az, kd);
