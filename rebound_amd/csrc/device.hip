@@ -205,6 +205,7 @@ void device_release(struct reb_simulation* r) {
     d->scratch.release();
     d->aos.release();
     d->flags.release();
+    d->drift_back.release();
     if (d->host_stage) (void)hipHostFree(d->host_stage);
     d->host_stage = nullptr;
     for (auto& e : d->kev)

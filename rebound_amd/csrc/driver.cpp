@@ -14,6 +14,7 @@
 using namespace rbamd;
 
 extern "C" void rb_whfast_step(struct reb_simulation* r, void* state);
+extern "C" void rb_leapfrog_step(struct reb_simulation* r, void* state);
 
 static volatile sig_atomic_t g_sigint = 0;
 static void sigint_handler(int signum) {
@@ -123,14 +124,15 @@ static void count_steps(struct reb_simulation* const r, const struct timeval& t0
     r->steps_done += n;
 }
 
-// Whether nothing on the host looks at the simulation between its WHFast
-// steps, so that several can run in one launch: no callback, exit check,
+// Whether nothing on the host looks at the simulation between two steps, so that
+// several WHFast steps can run in one launch and a leapfrog step can take the next
+// one's opening drift with its own closing one: no callback, exit check,
 // boundary, collision search, archive or variational set (whose rescaling and
 // MEGNO sums are formed on the host after every step).
 static bool steps_unobserved(const struct reb_simulation* r) {
-    return r->integrator.callbacks.step == rb_whfast_step && !r->heartbeat && !r->pre_timestep_modifications &&
-           !r->post_timestep_modifications && !r->additional_forces && !r->exit_max_distance &&
-           !r->exit_min_distance && !r->simulationarchive_filename && r->boundary == REB_BOUNDARY_NONE &&
+    return !r->heartbeat && !r->pre_timestep_modifications && !r->post_timestep_modifications &&
+           !r->additional_forces && !r->exit_max_distance && !r->exit_min_distance &&
+           !r->simulationarchive_filename && r->boundary == REB_BOUNDARY_NONE &&
            r->collision == REB_COLLISION_NONE && !r->N_odes && !r->N_var && r->usleep <= 0;
 }
 
@@ -143,7 +145,7 @@ static constexpr size_t kLaunchSteps = 1000;
 // takes 9 us on the device.  Returns the steps done, 0 when the caller has to
 // step one by one.  A refused launch counts as one step, as a refused step does.
 static size_t whfast_steps_at_once(struct reb_simulation* const r, size_t n) {
-    if (n < 2 || !steps_unobserved(r)) return 0;
+    if (n < 2 || r->integrator.callbacks.step != rb_whfast_step || !steps_unobserved(r)) return 0;
     struct timeval t0;
     gettimeofday(&t0, nullptr);
     if (!whfast_steps_device(r, (struct reb_integrator_whfast_state*)r->integrator.state, (long)n)) n = 1;
@@ -191,6 +193,15 @@ static void reb_simulation_step(struct reb_simulation* const r) {
     count_steps(r, t0, 1);
 }
 
+// Takes back an opening drift whose step does not come.
+static void end_steps(struct reb_simulation* r) {
+    DeviceState* d = dev_of(r);
+    d->step_follows = false;
+    if (!d->drifted_ahead) return;
+    d->drifted_ahead = false;
+    gravity_undo_drift(r);
+}
+
 // simulation.c:291-369
 static int reb_check_exit(struct reb_simulation* const r, const double tmax, double* last_full_dt) {
     if (r->status <= REB_STATUS_SINGLE_STEP) {
@@ -199,6 +210,7 @@ static int reb_check_exit(struct reb_simulation* const r, const double tmax, dou
         else
             r->status = (enum REB_STATUS)(r->status + 1);
     }
+    if (r->status == REB_STATUS_PAUSED || r->status == REB_STATUS_SCREENSHOT) end_steps(r);
     while (r->status == REB_STATUS_PAUSED || r->status == REB_STATUS_SCREENSHOT) {
         usleep(1000);
         if (g_sigint) r->status = REB_STATUS_SIGINT;
@@ -241,13 +253,13 @@ static int reb_check_exit(struct reb_simulation* const r, const double tmax, dou
 }
 
 // Steps of the present dt until reb_check_exit would do more than go on, with
-// the time advanced as the steps advance it; at most kLaunchSteps.
-static size_t steps_before_exit(const struct reb_simulation* r, double tmax) {
+// the time advanced as the steps advance it; at most `most`.
+static size_t steps_before_exit(const struct reb_simulation* r, double tmax, size_t most) {
     if (r->status != REB_STATUS_RUNNING) return 0;
     const double sign = copysign(1., r->dt);
     double t = r->t;
     size_t n = 0;
-    while (n < kLaunchSteps) {
+    while (n < most) {
         if (tmax != INFINITY) {
             const double ahead = r->exact_finish_time == 1 ? t + r->dt : t;
             if (ahead * sign >= tmax * sign) break;
@@ -257,6 +269,12 @@ static size_t steps_before_exit(const struct reb_simulation* r, double tmax) {
         n++;
     }
     return n;
+}
+
+// Tells the leapfrog whether, as far as can be known, another unobserved step of
+// the same dt follows the coming one.
+static void announce_step(struct reb_simulation* r, bool more) {
+    dev_of(r)->step_follows = more && r->integrator.callbacks.step == rb_leapfrog_step && steps_unobserved(r);
 }
 
 static void begin_call(struct reb_simulation* r) {
@@ -295,9 +313,11 @@ REB_API void reb_simulation_steps(struct reb_simulation* const r, size_t N_steps
             continue;
         }
         if (r->simulationarchive_filename) archive_heartbeat(r);
+        announce_step(r, i + 1 < N_steps);
         reb_simulation_step(r);
         run_heartbeat(r);
     }
+    end_steps(r);
     reb_simulation_synchronize(r);
     if (r->simulationarchive_filename) archive_heartbeat(r);
     end_call(r);
@@ -326,17 +346,19 @@ REB_API enum REB_STATUS reb_simulation_integrate(struct reb_simulation* const r,
     if (r->status != REB_STATUS_PAUSED && r->status != REB_STATUS_SCREENSHOT) r->status = REB_STATUS_RUNNING;
     run_heartbeat(r);
     while (reb_check_exit(r, tmax, &last_full_dt) < 0) {
-        const size_t k = whfast_steps_at_once(r, steps_before_exit(r, tmax));
+        const size_t k = whfast_steps_at_once(r, steps_before_exit(r, tmax, kLaunchSteps));
         if (k) {
             if (g_sigint) r->status = REB_STATUS_SIGINT;
             continue;
         }
         if (r->simulationarchive_filename) archive_heartbeat(r);
+        announce_step(r, steps_before_exit(r, tmax, 2) == 2);
         reb_simulation_step(r);
         run_heartbeat(r);
         if (g_sigint) r->status = REB_STATUS_SIGINT;
         if (r->usleep > 0) usleep((useconds_t)r->usleep);
     }
+    end_steps(r);
     reb_simulation_synchronize(r);
     if (r->exact_finish_time == 1) r->dt = last_full_dt;
     if (r->simulationarchive_filename) archive_heartbeat(r);

@@ -73,12 +73,50 @@ struct GBZero {
 };
 
 // The leapfrog's kick and closing drift, applied by the pass that finishes the
-// accelerations (on == 0: nothing).
+// accelerations (on == 0: nothing).  on == 2: the next step's opening drift
+// follows as well (a launch of 2 to 3 us less per step), the positions between the
+// two are kept in `back` (stride doubles per component) in case that step is not taken.
 struct KickDrift {
     double *x, *y, *z, *vx, *vy, *vz;
     double kick, drift;
     int on;
+    double* back;
+    size_t stride;
 };
+// What it reads, fetched before the accelerations are known.
+struct KickState {
+    double x, y, z, vx, vy, vz;
+};
+__device__ __forceinline__ KickState kick_load(const KickDrift& kd, int i) {
+    if (!kd.on) return KickState{};
+    return KickState{kd.x[i], kd.y[i], kd.z[i], kd.vx[i], kd.vy[i], kd.vz[i]};
+}
+// integrator_leapfrog.c:84-93 then :72-82: v += dt*a, x += dt/2*v (twice: the
+// next step's)
+__device__ __forceinline__ void kick_store(const KickDrift& kd, int i, const KickState& s, double ax, double ay,
+                                           double az) {
+    if (!kd.on) return;
+    const double vx = s.vx + kd.kick * ax;
+    const double vy = s.vy + kd.kick * ay;
+    const double vz = s.vz + kd.kick * az;
+    kd.vx[i] = vx;
+    kd.vy[i] = vy;
+    kd.vz[i] = vz;
+    double x = s.x + kd.drift * vx;
+    double y = s.y + kd.drift * vy;
+    double z = s.z + kd.drift * vz;
+    if (kd.on == 2) {
+        kd.back[i] = x;
+        kd.back[kd.stride + i] = y;
+        kd.back[2 * kd.stride + i] = z;
+        x += kd.drift * vx;
+        y += kd.drift * vy;
+        z += kd.drift * vz;
+    }
+    kd.x[i] = x;
+    kd.y[i] = y;
+    kd.z[i] = z;
+}
 
 __device__ __forceinline__ bool skip_pair(int i, int j, int ignore) {
     if (ignore == 1 && ((j == 1 && i == 0) || (i == 1 && j == 0))) return true;
@@ -107,9 +145,10 @@ __device__ __forceinline__ void kahan_add(double term, double& a, double& c) {
 // ascending source order: the reference's sequential sum, each component its own
 // chain.  The rows are double-buffered, so one barrier per tile suffices.  Small N
 // is bound by the chains (N dependent additions), so the summing lanes read their row
-// sixteen terms ahead.  1024 bodies 27 -> 17 us with the terms and the sums on
-// separate wavefronts and these reads; staging the sources in LDS four tiles ahead
-// gained nothing there and lost 15 % from 8192 bodies (fewer workgroups per CU).
+// sixteen terms ahead; the term threads load their sources two tiles ahead (staging
+// them in LDS lost 15 % from 8192 bodies: fewer workgroups per CU).  A leapfrog step
+// with the terms and the sums on the same wavefronts and now: 64 bodies 16.1 -> 11.3 us,
+// 1024 32.3 -> 22.0, 8192 231 -> 181, 32768 3.16 -> 2.7 ms.
 static constexpr int kExTermThreads = 256;
 static constexpr int kExThreads = kExTermThreads + 64;
 
@@ -568,16 +607,21 @@ __device__ __forceinline__ void direct_fast_block(const double* __restrict__ x, 
     double cx = 0., cy = 0., cz = 0.;      // Kahan carries (COMP per pair, FP64/SPLIT per tile)
     const double c15 = vreg_const(1.5);
     const double c1875 = vreg_const(1.875);
+    // the next tile's source of this thread, fetched a tile ahead (the first with
+    // the targets, not after a barrier that waits for them)
+    auto source = [&](int t) {
+        const int jj = t + (int)threadIdx.x;
+        return jj < j1 ? make_double4(x[jj], y[jj], z[jj], m[jj]) : make_double4(0., 0., 0., 0.);
+    };
+    double4 ahead = source(j0);
     for (int g = 0; g < gbs.n(); g++) {
         const GB3 gb = gbs.get(g);
         const double gx = gb.x + xi, gy = gb.y + yi, gz = gb.z + zi;
         for (int t = j0; t < j1; t += kFast) {
             __syncthreads();
-            const int jj = t + (int)threadIdx.x;
-            if (jj < j1) {
-                tile[threadIdx.x] = make_double4(x[jj], y[jj], z[jj], m[jj]);
-            }
+            tile[threadIdx.x] = ahead;
             __syncthreads();
+            ahead = source(t + kFast < j1 ? t + kFast : j0);
             const int n = min(kFast, j1 - t);
             // Only tiles holding a target of this block, or sources 0/1 when
             // terms are ignored, need the per-pair skip test (target 0 with
@@ -632,14 +676,14 @@ __global__ __launch_bounds__(kFast) __attribute__((amdgpu_waves_per_eu(RB_FAST_W
 // Sum the chunk partials in chunk order (Kahan), apply -G and write (or add to)
 // the acceleration.  ignore==2 zeroes particle 0 (it feels nothing).  With
 // kd.on, the leapfrog's kick and closing drift follow in the same pass
-// (integrator_leapfrog.c:84-93 then :72-82: v += dt*a, then x += dt/2*v),
-// which is safe because every read of the positions has finished.
+// (kick_store), which is safe because every read of the positions has finished.
 __device__ __forceinline__ void reduce_one(const double* __restrict__ partial, int pstride, int nchunk, int i,
                                            double negG, int accumulate, int ignore, double* __restrict__ ax,
                                            double* __restrict__ ay, double* __restrict__ az, const KickDrift& kd) {
     // Per component, chunk by chunk: the chunk's sum, then its carry with the
     // sign flipped, Kahan-added in chunk order.  The loads of eight chunks are
     // issued before their additions, so their latencies overlap.
+    const KickState ks = kick_load(kd, i);
     double s[3] = {0., 0., 0.}, k[3] = {0., 0., 0.};
     constexpr int B = 8;
     int q = 0;
@@ -678,17 +722,7 @@ __device__ __forceinline__ void reduce_one(const double* __restrict__ partial, i
     ax[i] = out[0];
     ay[i] = out[1];
     az[i] = out[2];
-    if (kd.on) {
-        const double vx = kd.vx[i] + kd.kick * out[0];
-        const double vy = kd.vy[i] + kd.kick * out[1];
-        const double vz = kd.vz[i] + kd.kick * out[2];
-        kd.vx[i] = vx;
-        kd.vy[i] = vy;
-        kd.vz[i] = vz;
-        kd.x[i] = kd.x[i] + kd.drift * vx;
-        kd.y[i] = kd.y[i] + kd.drift * vy;
-        kd.z[i] = kd.z[i] + kd.drift * vz;
-    }
+    kick_store(kd, i, ks, out[0], out[1], out[2]);
 }
 
 __global__ void k_reduce(const double* __restrict__ partial, int pstride, int nchunk, int n_recv, double negG,
@@ -704,15 +738,17 @@ __global__ void k_kick_drift(const double* __restrict__ ax, const double* __rest
                              const double* __restrict__ az, int n, KickDrift kd) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double vx = kd.vx[i] + kd.kick * ax[i];
-    const double vy = kd.vy[i] + kd.kick * ay[i];
-    const double vz = kd.vz[i] + kd.kick * az[i];
-    kd.vx[i] = vx;
-    kd.vy[i] = vy;
-    kd.vz[i] = vz;
-    kd.x[i] = kd.x[i] + kd.drift * vx;
-    kd.y[i] = kd.y[i] + kd.drift * vy;
-    kd.z[i] = kd.z[i] + kd.drift * vz;
+    kick_store(kd, i, kick_load(kd, i), ax[i], ay[i], az[i]);
+}
+
+// The positions before an opening drift that was taken ahead.
+__global__ void k_undo_drift(double* __restrict__ x, double* __restrict__ y, double* __restrict__ z,
+                             const double* __restrict__ back, size_t stride, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    x[i] = back[i];
+    y[i] = back[stride + i];
+    z[i] = back[2 * stride + i];
 }
 
 __global__ void k_zero3(double* __restrict__ a, double* __restrict__ b, double* __restrict__ c, int n) {
@@ -762,7 +798,7 @@ __global__ __launch_bounds__(256) void k_seg_reduce(const SegJob* __restrict__ j
     const SegJob J = jobs[R.job];
     const int i = R.first + (int)threadIdx.x;
     if (i >= J.n) return;
-    const KickDrift kd{J.x, J.y, J.z, J.vx, J.vy, J.vz, J.kick, J.drift, 1};
+    const KickDrift kd{J.x, J.y, J.z, J.vx, J.vy, J.vz, J.kick, J.drift, 1, nullptr, 0};
     reduce_one(J.partial, J.n, J.nchunk, i, J.negG, 0, 0, J.ax, J.ay, J.az, kd);
 }
 
@@ -1024,6 +1060,7 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
     const int i = first + lane;
     const int X = first / kSymSB, loc = first % kSymSB;
     const int ii = min(i, N - 1) - first;          // lanes past the end read the last body's
+    const KickState ks = w == 0 ? kick_load(kd, min(i, N - 1)) : KickState{};
     double s[3] = {0., 0., 0.}, c[3] = {0., 0., 0.};
     constexpr int PER = CARRY ? 2 : 1;             // entries per partial sum: itself, its carry
     const int total = PER * X + 2 * kSymDiag + PER * (nsb - 1 - X) * split;
@@ -1086,17 +1123,7 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
     ax[i] = o0;
     ay[i] = o1;
     az[i] = o2;
-    if (kd.on) {
-        const double vx = kd.vx[i] + kd.kick * o0;
-        const double vy = kd.vy[i] + kd.kick * o1;
-        const double vz = kd.vz[i] + kd.kick * o2;
-        kd.vx[i] = vx;
-        kd.vy[i] = vy;
-        kd.vz[i] = vz;
-        kd.x[i] = kd.x[i] + kd.drift * vx;
-        kd.y[i] = kd.y[i] + kd.drift * vy;
-        kd.z[i] = kd.z[i] + kd.drift * vz;
-    }
+    kick_store(kd, i, ks, o0, o1, o2);
 }
 
 // Superblock layout of the symmetric path for N bodies.
@@ -1387,9 +1414,29 @@ bool gravity_zero(struct reb_simulation* r) {
     return RB_HIP(r, hipGetLastError());
 }
 
+// Room for the positions that gravity_direct(.., ahead) keeps.  Without it the
+// step is taken as a single one.
+bool gravity_drift_room(struct reb_simulation* r) {
+    DeviceState* d = dev_of(r);
+    if (d->drift_back.ensure(sizeof(double) * 3 * d->cap)) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+// Back to the positions before the opening drift that the last step took ahead.
+bool gravity_undo_drift(struct reb_simulation* r) {
+    DeviceState* d = dev_of(r);
+    const int N = (int)r->N;
+    hipLaunchKernelGGL(k_undo_drift, dim3((N + 255) / 256), dim3(256), 0, d->stream, d->field(FX), d->field(FY),
+                       d->field(FZ), d->drift_back.as<double>(), d->cap, N);
+    mark_device_newer(r);
+    return RB_HIP(r, hipGetLastError());
+}
+
 // kick_drift (optional): {kick dt, drift dt} of a leapfrog step, applied in the
-// pass that finishes the accelerations.
-bool gravity_direct(struct reb_simulation* r, bool compensated, const double* kick_drift) {
+// pass that finishes the accelerations; ahead: and the same drift once more, the
+// next step's opening one.
+bool gravity_direct(struct reb_simulation* r, bool compensated, const double* kick_drift, bool ahead) {
     DeviceState* d = dev_of(r);
     const int N = (int)r->N;
     if (N == 0) return true;
@@ -1424,7 +1471,7 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
     KickDrift kd{};
     if (kick_drift) {
         kd = KickDrift{d->field(FX), d->field(FY), d->field(FZ), d->field(FVX), d->field(FVY), d->field(FVZ),
-                       kick_drift[0], kick_drift[1], 1};
+                       kick_drift[0], kick_drift[1], ahead ? 2 : 1, d->drift_back.as<double>(), d->cap};
     }
     // Every body active, no ghost boxes, nothing ignored: each pair once
     // (Newton's third law); otherwise the one-sided kernels.

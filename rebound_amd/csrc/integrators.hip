@@ -324,10 +324,17 @@ void rb_leapfrog_step(struct reb_simulation* r, void* state) {
                       !r->additional_forces && !dev_of(r)->dev_forces && !r->N_var && r->N > 0;
     switch (lf->order) {
         case 2:
-            D(dt * 0.5);
+            if (dev_of(r)->drifted_ahead) {
+                dev_of(r)->drifted_ahead = false;
+                r->t += dt * 0.5;
+            } else {
+                D(dt * 0.5);
+            }
             if (fuse) {
                 const double kd[2] = {dt, dt * 0.5};
-                if (!gravity_direct(r, r->gravity == REB_GRAVITY_COMPENSATED, kd)) return;
+                const bool ahead = dev_of(r)->step_follows && gravity_drift_room(r);
+                if (!gravity_direct(r, r->gravity == REB_GRAVITY_COMPENSATED, kd, ahead)) return;
+                dev_of(r)->drifted_ahead = ahead;
                 r->t += dt * 0.5;  // integrator_leapfrog.c:81
                 mark_device_newer(r);
             } else {

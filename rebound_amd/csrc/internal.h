@@ -131,6 +131,10 @@ struct DeviceState {
     std::vector<int2> sym_tasks_host;
     const void* sym_tasks_dev = nullptr;
     int sym_tasks_n = -1;
+    // leapfrog: the driver will take another step at once, unobserved; the last
+    // step's reduction took that step's opening drift (positions before it kept)
+    bool step_follows = false, drifted_ahead = false;
+    DevBuf drift_back;
     // ordered pairs evaluated by the timed pair kernels since the last read
     double kpairs = 0.;
     double* field(int f) const { return soa.as<double>() + (size_t)f * cap; }
@@ -161,7 +165,10 @@ std::vector<struct reb_vec6d> ghostboxes(struct reb_simulation* r, int nx, int n
 
 // ------------------------------------------------------------------ kernels (launchers)
 // Direct O(N^2) gravity (gravity.c:167-531) on the simulation's device state.
-bool gravity_direct(struct reb_simulation* r, bool compensated, const double* kick_drift = nullptr);
+bool gravity_direct(struct reb_simulation* r, bool compensated, const double* kick_drift = nullptr,
+                    bool ahead = false);
+bool gravity_drift_room(struct reb_simulation* r);
+bool gravity_undo_drift(struct reb_simulation* r);
 // The pair-symmetric direct-gravity path (gravity.hip) for N bodies, all
 // active, no ghost boxes, nothing ignored; its workspace in bytes.
 bool gravity_symmetric_path(size_t N, int precision);

@@ -216,7 +216,10 @@ static size_t nbody_footprint(size_t n, int precision, int gravity, bool least =
         else if (!compensated)
             ws = std::max(ws, gravity_symmetric_bytes_unsplit(n));
     }
-    return NFIELD * cap * sizeof(double) + ws + 16 * n + 4096;
+    // stepped alone: the positions before a drift taken ahead
+    const bool single = precision == REB_AMD_PRECISION_EXACT || gravity_symmetric_path(n, precision);
+    const size_t fields = NFIELD + (single && !least ? 3 : 0);
+    return fields * cap * sizeof(double) + ws + 16 * n + 4096;
 }
 
 // Jobs that run as single simulations on the worker threads: EXACT, and those
