@@ -1041,11 +1041,21 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
     }
 }
 
+// Adds the two-term number (hi, lo) to (s, c); exact in s whichever is larger,
+// where a Kahan addition rounds when the addend is the larger one.
+__device__ __forceinline__ void two_add(double hi, double lo, double& s, double& c) {
+    const double t = s + hi;
+    const double b = t - s;
+    c += ((s - (t - b)) + (hi - b)) + lo;
+    s = t;
+}
+
 // Per body: the partials of every superblock in ascending order (Kahan), then
 // -G and the fused kick and drift as in the one-sided reduction.  A workgroup
 // takes 64 bodies of one superblock; its four wavefronts each sum a quarter of
 // the partials (the loads of eight in flight), and the first adds the four
-// sums in order.  A body of superblock X has X source-side sums, kSymDiag one-sided
+// sums with their carries in order, as two-term numbers (any of the four can be the
+// largest).  A body of superblock X has X source-side sums, kSymDiag one-sided
 // sums with their carries, and `split` target-side sums per later superblock; CARRY: the
 // others come with carries too (COMPENSATED).
 template <bool CARRY>
@@ -1113,12 +1123,12 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
     __syncthreads();
     if (w != 0 || i >= N) return;
 #pragma unroll
-    for (int g = 1; g < 4; g++)
+    for (int f = 0; f < 3; f++) {
+        c[f] = -c[f];
 #pragma unroll
-        for (int f = 0; f < 3; f++) {
-            kahan_add(sums[g][f][lane], s[f], c[f]);
-            kahan_add(-sums[g][f + 3][lane], s[f], c[f]);
-        }
+        for (int g = 1; g < 4; g++) two_add(sums[g][f][lane], -sums[g][f + 3][lane], s[f], c[f]);
+        s[f] += c[f];
+    }
     const double o0 = negG * s[0], o1 = negG * s[1], o2 = negG * s[2];
     ax[i] = o0;
     ay[i] = o1;
@@ -1615,13 +1625,6 @@ __global__ __launch_bounds__(64) void k_energy_fold_terms(const double* __restri
 // triangle row the first one set the time (65536 bodies 12.5 ms, 10007 1.94, 1024 0.216;
 // now 1.80, 0.084 and 0.047, the call's copy and wait included).  A lane whose sum is NaN (coincident, non-finite or
 // overflowing distances) repeats its tile with IEEE arithmetic.
-__device__ __forceinline__ void two_add(double hi, double lo, double& s, double& c) {
-    const double t = s + hi;
-    const double b = t - s;
-    c += ((s - (t - b)) + (hi - b)) + lo;
-    s = t;
-}
-
 // Sum of (s, c) over the workgroup's threads into out[0] (sum) and out[1] (its
 // rounding error), in a fixed order.
 template <int THREADS>
