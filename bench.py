@@ -308,7 +308,7 @@ def ensemble_leg(amd, args):
             fl = oracle.whfast_flops_per_system_step(nb[:k], st[:int(nb[:k].sum())], dt[:k], 200)
             achieved = fl * res["value"] / 1e12
             res["roofline"] = {"bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                               "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_whfast_dh",
+                               "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_lane_dh",
                                "flop_per_system_step": fl,
                                "note": "latency-bound: 1.3 wavefronts per SIMD at 16384 systems"}
             log("ensemble cpu: %.3e system-steps/s on %d threads -> GPU %.0fx; energy errors match: %s" % (

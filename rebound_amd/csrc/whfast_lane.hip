@@ -4,7 +4,7 @@
 // kernels, the symplectic correctors, BASIC or COMPENSATED gravity, and at most
 // one first-order variational set (with or without MEGNO).  Test particles,
 // the kernels with Jacobi gravity and several variational sets run in the
-// general kernels of whfast.hip.
+// general kernels of whfast_general.hip.
 //
 // Reference: integrator_whfast.c:392-490, 612-784, 1051-1259, gravity.c:215-343
 // and :533-640, transformations.c:34-258 and :388-477, tools.c:1313-1380 and
