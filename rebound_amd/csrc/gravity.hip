@@ -840,8 +840,22 @@ __device__ __forceinline__ double dpp_ror1(double v) {
     return __hiloint2double(hi, lo);
 }
 
+// Tasks row by row: (0,1) (0,2) .. (0,nsb-1) (1,2) ..
 __host__ __device__ __forceinline__ int sym_task(int A, int B, int nsb) {
     return A * nsb - A * (A + 1) / 2 + (B - A - 1);
+}
+
+// The pair (A, B) of task t: the root of the row starts' quadratic, corrected in
+// integers.  Formed by every workgroup (a few hundred cycles of a 14 us part) and
+// not read from a list: a list would share its memory with the partial sums of the
+// other paths, or have to be kept in step with them.
+__host__ __device__ __forceinline__ int2 sym_pair(int t, int nsb) {
+    const double q = 2. * nsb - 1.;
+    int A = (int)((q - sqrt(q * q - 8. * t)) * 0.5);
+    A = A < 0 ? 0 : (A > nsb - 2 ? nsb - 2 : A);
+    while (A > 0 && sym_task(A, A + 1, nsb) > t) A--;
+    while (A < nsb - 2 && sym_task(A + 1, A + 2, nsb) <= t) A++;
+    return make_int2(A, A + 1 + t - sym_task(A, A + 1, nsb));
 }
 
 // Sums of three components; COMPENSATED gravity carries their Kahan corrections.
@@ -919,8 +933,8 @@ template <int MODE>
 __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, const double* __restrict__ m,
                                                     int N, int nsb, int ntasks, int split, double soft2,
-                                                    const int2* __restrict__ tasks, double* __restrict__ ipart,
-                                                    double* __restrict__ jpart, double* __restrict__ dpart) {
+                                                    double* __restrict__ ipart, double* __restrict__ jpart,
+                                                    double* __restrict__ dpart) {
     // J-block sources (x, y, z, m), double-buffered, each stored twice in a
     // row so that lane k reads entry k + 64 - s at step s without wrapping
     __shared__ double4 jt[2][2 * kSymJB];
@@ -937,10 +951,10 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
                                 u % kSymDiag, &jt[0][0]);
         return;
     }
-    const int2 tk = tasks[blockIdx.x % ntasks];
+    const int t = (int)blockIdx.x % ntasks;
     const int part = (int)blockIdx.x / ntasks;
-    const int A = tk.x, B = tk.y;
-    const int t = sym_task(A, B, nsb);
+    const int2 tk = sym_pair(t, nsb);
+    const int A = __builtin_amdgcn_readfirstlane(tk.x), B = __builtin_amdgcn_readfirstlane(tk.y);
     const int w = tid >> 6, k = tid & 63;
     // targets of this lane (A < B: never the ragged superblock)
     double tx[kSymTPL], ty[kSymTPL], tz[kSymTPL], tm[kSymTPL];
@@ -1141,7 +1155,7 @@ struct SymPlan {
     int nsb = 0;          // superblocks
     int ntasks = 0;       // superblock pairs A < B
     int split = 1;        // workgroups per task
-    size_t ipart_off = 0, jpart_off = 0, dpart_off = 0, tasks_off = 0, bytes = 0;   // workspace layout (bytes)
+    size_t ipart_off = 0, jpart_off = 0, dpart_off = 0, bytes = 0;   // workspace layout (bytes)
 };
 
 // Workgroups per task: the pair loop of a task takes about 223 us on a CU (its
@@ -1175,18 +1189,8 @@ static SymPlan sym_plan(int N, bool compensated) {
     p.ipart_off = 0;
     p.jpart_off = up(part * p.split);
     p.dpart_off = p.jpart_off + up(part);
-    p.tasks_off = p.dpart_off + up(sizeof(double) * 6 * kSymDiag * (size_t)N);
-    p.bytes = p.tasks_off + up(sizeof(int2) * (size_t)(p.ntasks > 0 ? p.ntasks : 1));
+    p.bytes = p.dpart_off + up(sizeof(double) * 6 * kSymDiag * (size_t)N);
     return p;
-}
-
-// The task list (A, B), A < B.
-static std::vector<int2> sym_tasks(const SymPlan& p) {
-    std::vector<int2> t;
-    t.reserve(p.ntasks);
-    for (int A = 0; A < p.nsb; A++)
-        for (int B = A + 1; B < p.nsb; B++) t.push_back(make_int2(A, B));
-    return t;
 }
 
 // Number of source chunks for the fast modes: chunks no shorter than kMinChunk
@@ -1254,7 +1258,7 @@ bool gravity_symmetric_path(size_t N, int precision) {
 size_t gravity_symmetric_bytes(size_t N, bool compensated) { return sym_plan((int)N, compensated).bytes; }
 size_t gravity_symmetric_bytes_unsplit(size_t N) {
     const size_t nsb = (N + kSymSB - 1) / kSymSB, tasks = nsb * (nsb - 1) / 2;
-    return tasks * (2 * 3 * sizeof(double) * kSymSB + sizeof(int2)) + 6 * sizeof(double) * N;
+    return tasks * 2 * 3 * sizeof(double) * kSymSB + 6 * sizeof(double) * N;
 }
 
 // Ordered pairs inside the superblocks (evaluated one-sided): sum over superblocks of n_A^2, self pairs included.
@@ -1271,14 +1275,13 @@ static int sym_launch(int mode, const double* x, const double* y, const double* 
     double* ipart = reinterpret_cast<double*>(base + plan.ipart_off);
     double* jpart = reinterpret_cast<double*>(base + plan.jpart_off);
     double* dpart = reinterpret_cast<double*>(base + plan.dpart_off);
-    const int2* tasks = reinterpret_cast<const int2*>(base + plan.tasks_off);
     const dim3 grid(plan.ntasks * plan.split + (N + kFast - 1) / kFast * kSymDiag);
     if (ev) (void)hipEventRecord(ev[0], st);
     const auto pairs = mode == FM_COMP    ? k_direct_sym<FM_COMP>
                        : mode == FM_SPLIT ? k_direct_sym<FM_SPLIT>
                                           : k_direct_sym<FM_FP64>;
-    hipLaunchKernelGGL(pairs, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks, plan.split, soft2, tasks,
-                       ipart, jpart, dpart);
+    hipLaunchKernelGGL(pairs, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks, plan.split, soft2, ipart,
+                       jpart, dpart);
     if (ev) (void)hipEventRecord(ev[1], st);
     const auto reduce = mode == FM_COMP ? k_sym_reduce<true> : k_sym_reduce<false>;
     hipLaunchKernelGGL(reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb, plan.split, -G,
@@ -1493,15 +1496,6 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
             return false;
         }
         char* base = static_cast<char*>(d->partial.p);
-        int2* tasks = reinterpret_cast<int2*>(base + plan.tasks_off);
-        if (d->sym_tasks_n != N || d->sym_tasks_dev != (const void*)tasks) {
-            d->sym_tasks_host = sym_tasks(plan);
-            if (!RB_HIP(r, hipMemcpyAsync(tasks, d->sym_tasks_host.data(), sizeof(int2) * d->sym_tasks_host.size(),
-                                          hipMemcpyHostToDevice, d->stream)))
-                return false;
-            d->sym_tasks_n = N;
-            d->sym_tasks_dev = tasks;
-        }
         if (d->profiling) d->kpairs += (double)N * (double)N - sym_diag_pairs(N);
         const int mode = seg_fast_mode(d->precision, compensated);
         const int rc = sym_launch(mode, d->field(FX), d->field(FY), d->field(FZ), d->field(FM), d->field(FAX),

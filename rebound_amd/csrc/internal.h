@@ -126,11 +126,6 @@ struct DeviceState {
     void* dev_forces_user = nullptr;
     // the EXACT energy fell back to the compensated sum once (warned)
     bool warned_energy_exact = false;
-    // task list of the symmetric direct-gravity path: for N bodies, at this
-    // device address inside `partial`
-    std::vector<int2> sym_tasks_host;
-    const void* sym_tasks_dev = nullptr;
-    int sym_tasks_n = -1;
     // leapfrog: the driver will take another step at once, unobserved; the last
     // step's reduction took that step's opening drift (positions before it kept)
     bool step_follows = false, drifted_ahead = false;
