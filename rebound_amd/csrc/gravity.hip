@@ -21,6 +21,7 @@
 // Data layout: structure of arrays (x, y, z, m as separate double arrays).
 // Sources are staged per 256-wide tile into LDS as double4 (x, y, z, m) and
 // read back as broadcasts (every lane of a wavefront reads the same entry).
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -818,12 +819,17 @@ __global__ __launch_bounds__(256) void k_seg_reduce(const SegJob* __restrict__ j
 // fused multiply-adds on each side; per step the rotation adds six moves.
 //
 // Outputs, all in fixed order (the results are deterministic):
-//   ipart[t][p][c][SB]  target-side sums of part p of task t (targets of A, sources of B)
-//   jpart[t][c][SB]  source-side sums of task t (bodies of B, all targets of A)
+//   ipart[t][p][c][SB]  target-side sums of part p of the launch's task t (targets of A, sources of B)
+//   jpart[t][c][SB]  source-side sums of the launch's task t (bodies of B, all targets of A)
 //                    with the sign of the term for A's bodies: S_j = -jpart
 //   dpart[d][6][N]   the one-sided sums within each superblock, 256 sources each (direct_fast_block)
 // and k_sym_reduce adds, per body, the partials of every superblock in
 // ascending order with Kahan compensation.
+//
+// ipart and jpart grow with the square of the body count (98 KB per task in
+// COMPENSATED gravity: 1.9 GB at 200000 bodies), so beyond a limit the tasks run in
+// several launches, in task order, each followed by a reduction that carries the
+// running sums of every body on to the next: the same additions in the same order.
 #ifndef RB_SYM_TPL
 #define RB_SYM_TPL 4
 #endif
@@ -831,6 +837,10 @@ static constexpr int kSymTPL = RB_SYM_TPL;           // targets per lane
 static constexpr int kSymSB = 4 * 64 * kSymTPL;       // bodies per superblock
 static constexpr int kSymJB = 64;                     // sources per J-block
 static constexpr int kSymMinN = 8192;                 // below: the one-sided kernel
+static constexpr size_t kSymMaxN = (size_t)kSymSB << 14;   // above: the same (task numbers in 32 bits)
+// Partial sums in memory at a time.  Several launches come from about 126000 bodies
+// (COMPENSATED: 88000), all but the last of at least 21 rounds of the chip.
+static constexpr size_t kSymPartials = (size_t)512 << 20;
 static constexpr int kSymDiag = kSymSB / kFast;       // source tiles of a superblock (one-sided pairs)
 
 // Lane k receives lane k-1's value, lane 0 lane 63's (DPP wave_ror:1).
@@ -922,17 +932,17 @@ __device__ __forceinline__ void sym_jblock(const double4* __restrict__ src, int 
     }
 }
 
-// Workgroups [0, ntasks * split): part p of task (A, B) takes 1/split of B's
+// Workgroups [0, ntasks * split): part p of task t0 + t, (A, B), takes 1/split of B's
 // J-blocks.  One workgroup per task leaves most of the chip idle below ~40000
 // bodies (8192 bodies are 28 tasks for 256 CUs), so sym_split cuts the tasks.
-// The remaining workgroups evaluate the pairs inside the superblocks
+// The remaining workgroups (of the first launch) evaluate the pairs inside the superblocks
 // (one-sided, 256 targets x 256 sources each); they are short and fill the
 // launch's tail.  One launch for full and ragged tasks alike (10007 bodies took
 // 237 + 221 us in two).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, const double* __restrict__ m,
-                                                    int N, int nsb, int ntasks, int split, double soft2,
+                                                    int N, int nsb, int t0, int ntasks, int split, double soft2,
                                                     double* __restrict__ ipart, double* __restrict__ jpart,
                                                     double* __restrict__ dpart) {
     // J-block sources (x, y, z, m), double-buffered, each stored twice in a
@@ -953,7 +963,7 @@ __global__ __launch_bounds__(256) void k_direct_sym(const double* __restrict__ x
     }
     const int t = (int)blockIdx.x % ntasks;
     const int part = (int)blockIdx.x / ntasks;
-    const int2 tk = sym_pair(t, nsb);
+    const int2 tk = sym_pair(t0 + t, nsb);
     const int A = __builtin_amdgcn_readfirstlane(tk.x), B = __builtin_amdgcn_readfirstlane(tk.y);
     const int w = tid >> 6, k = tid & 63;
     // targets of this lane (A < B: never the ragged superblock)
@@ -1072,10 +1082,16 @@ __device__ __forceinline__ void two_add(double hi, double lo, double& s, double&
 // largest).  A body of superblock X has X source-side sums, kSymDiag one-sided
 // sums with their carries, and `split` target-side sums per later superblock; CARRY: the
 // others come with carries too (COMPENSATED).
-template <bool CARRY>
+//
+// ROUNDS: after the launch of tasks t0 .. t1 - 1 of ntasks.  Tasks are numbered by rows
+// (A, A+1) (A, A+2) .., so a body's partials come in ascending order from launch to
+// launch; each wavefront continues its quarter from `state` (6 sums and carries of
+// N bodies per quarter), and the last launch's reduction ends as the only one does.
+template <bool CARRY, bool ROUNDS>
 __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ ipart,
                                                     const double* __restrict__ jpart,
                                                     const double* __restrict__ dpart, int N, int nsb, int split,
+                                                    int t0, int t1, int ntasks, double* __restrict__ state,
                                                     double negG, double* __restrict__ ax, double* __restrict__ ay,
                                                     double* __restrict__ az, KickDrift kd) {
     __shared__ double sums[4][6][64];
@@ -1084,11 +1100,34 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
     const int i = first + lane;
     const int X = first / kSymSB, loc = first % kSymSB;
     const int ii = min(i, N - 1) - first;          // lanes past the end read the last body's
-    const KickState ks = w == 0 ? kick_load(kd, min(i, N - 1)) : KickState{};
+    const bool last = !ROUNDS || t1 == ntasks;
+    if (!ROUNDS) t0 = 0;
+    const KickState ks = w == 0 && last ? kick_load(kd, min(i, N - 1)) : KickState{};
     double s[3] = {0., 0., 0.}, c[3] = {0., 0., 0.};
     constexpr int PER = CARRY ? 2 : 1;             // entries per partial sum: itself, its carry
     const int total = PER * X + 2 * kSymDiag + PER * (nsb - 1 - X) * split;
-    const int e0 = total * w / 4, e1 = total * (w + 1) / 4;
+    int e0 = total * w / 4, e1 = total * (w + 1) / 4;
+    if (ROUNDS) {
+        // entries of superblock X that the tasks before t complete (the one-sided
+        // ones count with the last source-side entry)
+        auto before = [&](int t) {
+            if (t == 0) return 0;
+            if (t == ntasks) return total;
+            const int2 next = sym_pair(t, nsb);
+            if (next.x < X) return PER * (next.x + (X < next.y ? 1 : 0));
+            return next.x > X ? total : PER * X + 2 * kSymDiag + PER * (next.y - X - 1) * split;
+        };
+        const int b0 = before(t0), b1 = before(t1);
+        if (b0 > e0 && i < N) {
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                s[f] = state[(size_t)(6 * w + f) * N + i];
+                c[f] = state[(size_t)(6 * w + 3 + f) * N + i];
+            }
+        }
+        e0 = max(e0, b0);
+        e1 = min(e1, b1);
+    }
     // entry e: base pointer of its first component, component stride, sign
     auto load = [&](int e, double* v) {
         const double* p;
@@ -1096,7 +1135,7 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
         double sign = 1.;
         if (e < PER * X) {
             const int carry = e % PER;
-            p = jpart + ((size_t)sym_task(e / PER, X, nsb) * 3 * PER + 3 * carry) * kSymSB + loc;
+            p = jpart + ((size_t)(sym_task(e / PER, X, nsb) - t0) * 3 * PER + 3 * carry) * kSymSB + loc;
             sign = carry ? 1. : -1.;
         } else if (e < PER * X + 2 * kSymDiag) {
             const int q = e - PER * X;
@@ -1105,7 +1144,7 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
             sign = q & 1 ? -1. : 1.;
         } else {
             const int q = (e - PER * X - 2 * kSymDiag) / PER, carry = (e - PER * X - 2 * kSymDiag) % PER;
-            const size_t part = (size_t)sym_task(X, X + 1 + q / split, nsb) * split + q % split;
+            const size_t part = (size_t)(sym_task(X, X + 1 + q / split, nsb) - t0) * split + q % split;
             p = ipart + (part * 3 * PER + 3 * carry) * kSymSB + loc;
             sign = carry ? -1. : 1.;
         }
@@ -1128,6 +1167,15 @@ __global__ __launch_bounds__(256) void k_sym_reduce(const double* __restrict__ i
         load(e, v);
 #pragma unroll
         for (int f = 0; f < 3; f++) kahan_add(v[f], s[f], c[f]);
+    }
+    if (!last) {
+        if (e0 >= e1 || i >= N) return;
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            state[(size_t)(6 * w + f) * N + i] = s[f];
+            state[(size_t)(6 * w + 3 + f) * N + i] = c[f];
+        }
+        return;
     }
 #pragma unroll
     for (int f = 0; f < 3; f++) {
@@ -1155,7 +1203,8 @@ struct SymPlan {
     int nsb = 0;          // superblocks
     int ntasks = 0;       // superblock pairs A < B
     int split = 1;        // workgroups per task
-    size_t ipart_off = 0, jpart_off = 0, dpart_off = 0, bytes = 0;   // workspace layout (bytes)
+    int round = 0;        // tasks per launch
+    size_t ipart_off = 0, jpart_off = 0, dpart_off = 0, state_off = 0, bytes = 0;   // workspace layout (bytes)
 };
 
 // Workgroups per task: the pair loop of a task takes about 223 us on a CU (its
@@ -1164,13 +1213,14 @@ struct SymPlan {
 // sums, about 12 ns of the chip's bandwidth.  The split with the least
 // modelled time; measured (leapfrog steps, FP64): 8192 bodies 59 us (286
 // unsplit), 10007 75 (526), 20000 210 (566), 24576 301 (513), 49152 965 (1200).
+static constexpr int kCUs = 256;
 static int sym_split(int ntasks) {
-    constexpr int kCUs = 256;
     constexpr double kTask = 223., kPart = 0.012;   // us
     int best = 1;
     double least = 1e300;
     for (int s = 1; s <= kSymSB / kSymJB; s *= 2) {
-        const double t = (ntasks * s + kCUs - 1) / kCUs * kTask / s + ntasks * s * kPart;
+        const long parts = (long)ntasks * s;
+        const double t = (parts + kCUs - 1) / kCUs * kTask / s + parts * kPart;
         if (t < least) {
             least = t;
             best = s;
@@ -1179,17 +1229,30 @@ static int sym_split(int ntasks) {
     return best;
 }
 
-static SymPlan sym_plan(int N, bool compensated) {
+// The plan whose workspace stays within `limit` bytes, or the least one if none
+// does: launches of a whole number of rounds of the chip, at least one (with fewer
+// workgroups the one-sided kernels are faster).
+static SymPlan sym_plan(int N, bool compensated, size_t limit) {
     SymPlan p;
     p.nsb = (N + kSymSB - 1) / kSymSB;
     p.ntasks = p.nsb * (p.nsb - 1) / 2;
     p.split = sym_split(p.ntasks);
-    const size_t part = sizeof(double) * (compensated ? 6 : 3) * (size_t)kSymSB * (size_t)p.ntasks;
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    p.ipart_off = 0;
-    p.jpart_off = up(part * p.split);
-    p.dpart_off = p.jpart_off + up(part);
-    p.bytes = p.dpart_off + up(sizeof(double) * 6 * kSymDiag * (size_t)N);
+    const size_t part = sizeof(double) * (compensated ? 6 : 3) * (size_t)kSymSB;
+    const size_t task = part * (p.split + 1);
+    const size_t dpart = up(sizeof(double) * 6 * kSymDiag * (size_t)N);
+    const size_t state = up(sizeof(double) * 24 * (size_t)N);
+    p.round = p.ntasks;
+    if (task * p.ntasks > kSymPartials || task * p.ntasks + dpart > limit) {
+        const size_t unit = kCUs / p.split;
+        const size_t room = limit > dpart + state ? std::min(limit - dpart - state, kSymPartials) : 0;
+        const size_t fit = std::max(room / task / unit, (size_t)1) * unit;
+        if (fit < (size_t)p.ntasks) p.round = (int)fit;
+    }
+    p.jpart_off = part * p.split * p.round;                    // multiples of 24 KB
+    p.dpart_off = p.jpart_off + part * p.round;
+    p.state_off = p.dpart_off + dpart;
+    p.bytes = p.state_off + (p.round < p.ntasks ? state : 0);
     return p;
 }
 
@@ -1253,9 +1316,11 @@ int seg_fast_mode(int precision, int compensated) {
 // ignored terms, takes the symmetric path in this precision and gravity, and
 // the workspace it then needs.
 bool gravity_symmetric_path(size_t N, int precision) {
-    return precision != REB_AMD_PRECISION_EXACT && N >= (size_t)kSymMinN;
+    return precision != REB_AMD_PRECISION_EXACT && N >= (size_t)kSymMinN && N <= kSymMaxN;
 }
-size_t gravity_symmetric_bytes(size_t N, bool compensated) { return sym_plan((int)N, compensated).bytes; }
+size_t gravity_symmetric_bytes(size_t N, bool compensated) {
+    return sym_plan((int)N, compensated, SIZE_MAX).bytes;
+}
 size_t gravity_symmetric_bytes_unsplit(size_t N) {
     const size_t nsb = (N + kSymSB - 1) / kSymSB, tasks = nsb * (nsb - 1) / 2;
     return tasks * 2 * 3 * sizeof(double) * kSymSB + 6 * sizeof(double) * N;
@@ -1267,25 +1332,31 @@ static double sym_diag_pairs(int N) {
     return (double)full * kSymSB * kSymSB + (double)rest * rest;
 }
 
-// One force evaluation on the symmetric path: all pairs (events around this
-// launch), then the per-body reduction with the fused kick and drift.
+// One force evaluation on the symmetric path: all pairs (events around these
+// launches), then the per-body reduction with the fused kick and drift.
 static int sym_launch(int mode, const double* x, const double* y, const double* z, const double* m, double* ax,
                       double* ay, double* az, int N, double G, double soft2, const SymPlan& plan, char* base,
                       hipStream_t st, hipEvent_t* ev, const KickDrift& kd) {
     double* ipart = reinterpret_cast<double*>(base + plan.ipart_off);
     double* jpart = reinterpret_cast<double*>(base + plan.jpart_off);
     double* dpart = reinterpret_cast<double*>(base + plan.dpart_off);
-    const dim3 grid(plan.ntasks * plan.split + (N + kFast - 1) / kFast * kSymDiag);
-    if (ev) (void)hipEventRecord(ev[0], st);
+    double* state = reinterpret_cast<double*>(base + plan.state_off);
     const auto pairs = mode == FM_COMP    ? k_direct_sym<FM_COMP>
                        : mode == FM_SPLIT ? k_direct_sym<FM_SPLIT>
                                           : k_direct_sym<FM_FP64>;
-    hipLaunchKernelGGL(pairs, grid, dim3(256), 0, st, x, y, z, m, N, plan.nsb, plan.ntasks, plan.split, soft2, ipart,
-                       jpart, dpart);
-    if (ev) (void)hipEventRecord(ev[1], st);
-    const auto reduce = mode == FM_COMP ? k_sym_reduce<true> : k_sym_reduce<false>;
-    hipLaunchKernelGGL(reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb, plan.split, -G,
-                       ax, ay, az, kd);
+    const bool rounds = plan.round < plan.ntasks;
+    const auto reduce = mode == FM_COMP ? (rounds ? k_sym_reduce<true, true> : k_sym_reduce<true, false>)
+                                        : (rounds ? k_sym_reduce<false, true> : k_sym_reduce<false, false>);
+    if (ev) (void)hipEventRecord(ev[0], st);
+    for (int t0 = 0; t0 < plan.ntasks; t0 += plan.round) {
+        const int t1 = std::min(t0 + plan.round, plan.ntasks);
+        const int inner = t0 == 0 ? (N + kFast - 1) / kFast * kSymDiag : 0;
+        hipLaunchKernelGGL(pairs, dim3((t1 - t0) * plan.split + inner), dim3(256), 0, st, x, y, z, m, N, plan.nsb, t0,
+                           t1 - t0, plan.split, soft2, ipart, jpart, dpart);
+        if (ev && t1 == plan.ntasks) (void)hipEventRecord(ev[1], st);
+        hipLaunchKernelGGL(reduce, dim3((N + 63) / 64), dim3(256), 0, st, ipart, jpart, dpart, N, plan.nsb, plan.split,
+                           t0, t1, plan.ntasks, state, -G, ax, ay, az, kd);
+    }
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -1490,18 +1561,24 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
     // (Newton's third law); otherwise the one-sided kernels.
     if (ngb == 1 && N_active == N && r->gravity_ignore_terms == 0 &&
         gravity_symmetric_path((size_t)N, d->precision)) {
-        const SymPlan plan = sym_plan(N, compensated);
-        if (!d->partial.ensure(plan.bytes)) {
-            reb_simulation_error(r, "Out of device memory for the gravity workspace.");
-            return false;
+        // The tasks go in as many launches as the memory asks for (the same bits);
+        // a simulation without room for even the shortest takes the one-sided
+        // kernels below.
+        for (;;) {
+            const SymPlan plan = sym_plan(N, compensated, d->sym_limit);
+            if (plan.bytes > d->sym_limit) break;
+            if (!d->partial.ensure(plan.bytes)) {
+                (void)hipGetLastError();
+                d->sym_limit = plan.bytes / 2;
+                continue;
+            }
+            if (d->profiling) d->kpairs += (double)N * (double)N - sym_diag_pairs(N);
+            const int rc = sym_launch(seg_fast_mode(d->precision, compensated), d->field(FX), d->field(FY),
+                                      d->field(FZ), d->field(FM), d->field(FAX), d->field(FAY), d->field(FAZ), N, r->G,
+                                      soft2, plan, static_cast<char*>(d->partial.p), d->stream, ev, kd);
+            if (rc) return RB_HIP(r, hipGetLastError());
+            return true;
         }
-        char* base = static_cast<char*>(d->partial.p);
-        if (d->profiling) d->kpairs += (double)N * (double)N - sym_diag_pairs(N);
-        const int mode = seg_fast_mode(d->precision, compensated);
-        const int rc = sym_launch(mode, d->field(FX), d->field(FY), d->field(FZ), d->field(FM), d->field(FAX),
-                                  d->field(FAY), d->field(FAZ), N, r->G, soft2, plan, base, d->stream, ev, kd);
-        if (rc) return RB_HIP(r, hipGetLastError());
-        return true;
     }
     const int nchunk = pick_chunks(N, N_active, ngb);
     if (!d->partial.ensure(workspace_bytes(N, nchunk) + 256)) {

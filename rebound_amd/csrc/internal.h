@@ -94,6 +94,7 @@ struct DeviceState {
     size_t cap = 0;                 // particle capacity of `soa`
     DevBuf soa;                     // NFIELD * cap doubles
     DevBuf partial;                 // j-split partial sums for direct gravity
+    size_t sym_limit = SIZE_MAX;    // most of it that the pair-symmetric path takes (bytes)
     DevBuf scratch;                 // small reductions (energy, flags)
     DevBuf aos;                     // AoS staging for uploads/downloads
     DevBuf flags;                   // device error words (boundary wrap)
