@@ -304,7 +304,10 @@ REB_API long reb_amd_server_submit_simulation(struct reb_amd_server* s, struct r
  * 0 on success, 1 (message in reb_amd_last_error) for an unknown or failed
  * job or a file that cannot be written.  No counterpart in the reference. */
 REB_API int reb_amd_server_checkpoint(struct reb_amd_server* s, long job, const char* filename);
-/* Device-memory footprint of a job, as admission counts it. */
+/* Device-memory footprint of a job, as admission counts it; for an N-body job
+ * under a budget that holds it whole.  A smaller budget still takes a large one
+ * (BASIC or COMPENSATED, 8192 bodies or more) if it fits with its pair sums in
+ * several launches, and charges it what it then allocates. */
 REB_API size_t reb_amd_server_whfast_bytes(size_t n_bodies);
 REB_API size_t reb_amd_server_nbody_bytes(size_t n, int precision);
 REB_API int reb_amd_server_status(struct reb_amd_server* s, long job);

@@ -1318,12 +1318,8 @@ int seg_fast_mode(int precision, int compensated) {
 bool gravity_symmetric_path(size_t N, int precision) {
     return precision != REB_AMD_PRECISION_EXACT && N >= (size_t)kSymMinN && N <= kSymMaxN;
 }
-size_t gravity_symmetric_bytes(size_t N, bool compensated) {
-    return sym_plan((int)N, compensated, SIZE_MAX).bytes;
-}
-size_t gravity_symmetric_bytes_unsplit(size_t N) {
-    const size_t nsb = (N + kSymSB - 1) / kSymSB, tasks = nsb * (nsb - 1) / 2;
-    return tasks * 2 * 3 * sizeof(double) * kSymSB + 6 * sizeof(double) * N;
+size_t gravity_symmetric_bytes(size_t N, bool compensated, size_t limit) {
+    return sym_plan((int)N, compensated, limit).bytes;
 }
 
 // Ordered pairs inside the superblocks (evaluated one-sided): sum over superblocks of n_A^2, self pairs included.
@@ -1498,10 +1494,11 @@ bool gravity_zero(struct reb_simulation* r) {
     return RB_HIP(r, hipGetLastError());
 }
 
-// Room for the positions that gravity_direct(.., ahead) keeps.  Without it the
-// step is taken as a single one.
+// Room for the positions that gravity_direct(.., ahead) keeps.  Without it, or
+// with limited memory, the step is taken as a single one.
 bool gravity_drift_room(struct reb_simulation* r) {
     DeviceState* d = dev_of(r);
+    if (d->sym_limit != SIZE_MAX) return false;
     if (d->drift_back.ensure(sizeof(double) * 3 * d->cap)) return true;
     (void)hipGetLastError();
     return false;

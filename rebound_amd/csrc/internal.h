@@ -94,7 +94,8 @@ struct DeviceState {
     size_t cap = 0;                 // particle capacity of `soa`
     DevBuf soa;                     // NFIELD * cap doubles
     DevBuf partial;                 // j-split partial sums for direct gravity
-    size_t sym_limit = SIZE_MAX;    // most of it that the pair-symmetric path takes (bytes)
+    // most of it that the pair-symmetric path takes (bytes); SIZE_MAX: memory is not short
+    size_t sym_limit = SIZE_MAX;
     DevBuf scratch;                 // small reductions (energy, flags)
     DevBuf aos;                     // AoS staging for uploads/downloads
     DevBuf flags;                   // device error words (boundary wrap)
@@ -166,12 +167,10 @@ bool gravity_direct(struct reb_simulation* r, bool compensated, const double* ki
 bool gravity_drift_room(struct reb_simulation* r);
 bool gravity_undo_drift(struct reb_simulation* r);
 // The pair-symmetric direct-gravity path (gravity.hip) for N bodies, all
-// active, no ghost boxes, nothing ignored; its workspace in bytes.
+// active, no ghost boxes, nothing ignored; its workspace in bytes when that is to
+// stay within `limit` (more than the limit: it cannot).
 bool gravity_symmetric_path(size_t N, int precision);
-size_t gravity_symmetric_bytes(size_t N, bool compensated);
-// What that workspace comes to without splitting tasks over workgroups or
-// carries: the least a job is charged for it.
-size_t gravity_symmetric_bytes_unsplit(size_t N);
+size_t gravity_symmetric_bytes(size_t N, bool compensated, size_t limit);
 
 // Batched order-2 leapfrog steps with direct gravity for many independent
 // simulations (gravity.hip k_seg_*).  A SegJob holds one simulation's device

@@ -27,7 +27,8 @@
 // they join and leave between rounds.  Jobs in EXACT precision, and jobs
 // large enough for the pair-symmetric force path (gravity.hip), run as single
 // simulations from worker threads on a third stream, so that every job's bits
-// are those of stepping it alone.  The streams overlap on the device.
+// are those of stepping it alone (but for a COMPENSATED job that the whole budget
+// holds only with the one-sided force, see nbody_memory).  The streams overlap on the device.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -68,6 +69,7 @@ struct Job {
     int safe_mode = 0, gravity = REB_GRAVITY_BASIC, precision = REB_AMD_PRECISION_FP64;
     uint64_t n_steps = 0;
     size_t footprint = 0;
+    size_t sym_limit = SIZE_MAX;   // N-body: see NbodyMemory
     int state = REB_AMD_JOB_PENDING;
     std::string error;
     double t_submit = 0., t_admit = 0., t_done = 0.;
@@ -202,24 +204,35 @@ static double since(const Server* S) {
 
 static size_t whfast_footprint(size_t n) { return n * 17 * sizeof(double) + sizeof(WHSys) + 64; }
 
-// least: with the force's smallest workspace, which decides whether a budget can
-// hold the job at all.  The larger workspaces of the fast paths are charged up to
-// the budget: a job that fits alone without them is not refused for them.
-static size_t nbody_footprint(size_t n, int precision, int gravity, bool least = false) {
+// What an N-body job allocates on the device, and the limit for its pair-symmetric
+// partial sums (gravity_symmetric_bytes) under which it allocates that.
+struct NbodyMemory {
+    size_t bytes, sym_limit;
+};
+
+// A job that fits the budget only in less memory than it takes alone runs in less:
+// without the drift taken ahead and with the pair-symmetric force in several
+// launches, which leaves its bits as they are; and a COMPENSATED one without room
+// for that with the one-sided kernels, whose last bits differ.  bytes > budget: the
+// job does not fit.
+static NbodyMemory nbody_memory(size_t n, int precision, int gravity, size_t budget) {
     size_t cap = 64;
     while (cap < n) cap *= 2;
-    size_t ws = reb_amd_gravity_workspace_bytes(n, precision);
+    const size_t state = NFIELD * cap * sizeof(double) + 16 * n + 4096;
+    const size_t one_sided = reb_amd_gravity_workspace_bytes(n, precision);
+    const bool symmetric = gravity_symmetric_path(n, precision);
     const bool compensated = gravity == REB_GRAVITY_COMPENSATED;
-    if (gravity_symmetric_path(n, precision)) {
-        if (!least)
-            ws = std::max(ws, gravity_symmetric_bytes(n, compensated));
-        else if (!compensated)
-            ws = std::max(ws, gravity_symmetric_bytes_unsplit(n));
-    }
-    // stepped alone: the positions before a drift taken ahead
-    const bool single = precision == REB_AMD_PRECISION_EXACT || gravity_symmetric_path(n, precision);
-    const size_t fields = NFIELD + (single && !least ? 3 : 0);
-    return fields * cap * sizeof(double) + ws + 16 * n + 4096;
+    if (!symmetric && precision != REB_AMD_PRECISION_EXACT) return {state + one_sided, SIZE_MAX};   // batched
+    // stepped alone: also the positions before a drift taken ahead
+    const size_t ahead = 3 * cap * sizeof(double);
+    const size_t whole =
+        state + ahead + (symmetric ? gravity_symmetric_bytes(n, compensated, SIZE_MAX) : one_sided);
+    if (whole <= budget) return {whole, SIZE_MAX};
+    const size_t room = budget > state ? budget - state : 0;
+    if (!symmetric) return {state + one_sided, 0};
+    const size_t part = gravity_symmetric_bytes(n, compensated, room);
+    if (part > room && compensated && one_sided <= room) return {state + one_sided, 0};
+    return {state + part, room};
 }
 
 // Jobs that run as single simulations on the worker threads: EXACT, and those
@@ -741,6 +754,7 @@ static void run_nbody(Server* S, Job* j, hipStream_t stream) {
     d->device = S->device;
     d->stream = stream;        // the worker's stream, kept by the server
     d->owns_stream = false;
+    d->sym_limit = j->sym_limit;
     r->save_messages = 1;
     r->G = j->G;
     r->softening = j->softening;
@@ -1178,9 +1192,11 @@ REB_API void reb_amd_server_free(struct reb_amd_server* h) {
 
 static long submit(Server* S, std::unique_ptr<Job> j) {
     std::lock_guard<std::mutex> g(S->mu);
-    if (j->kind == JOB_NBODY && j->footprint > S->budget &&
-        nbody_footprint(j->bodies.size(), j->precision, j->gravity, true) <= S->budget)
-        j->footprint = S->budget;
+    if (j->kind == JOB_NBODY) {
+        const NbodyMemory m = nbody_memory(j->bodies.size(), j->precision, j->gravity, S->budget);
+        j->footprint = m.bytes;
+        j->sym_limit = m.sym_limit;
+    }
     if (j->footprint > S->budget) {
         S->err = "job footprint (" + std::to_string(j->footprint) + " bytes) exceeds the memory budget";
         set_last_error(S->err);
@@ -1235,7 +1251,6 @@ REB_API long reb_amd_server_submit_nbody(struct reb_amd_server* h, size_t n, con
     j->n_steps = n_steps;
     j->gravity = gravity;
     j->precision = precision;
-    j->footprint = nbody_footprint(n, precision, gravity);
     return submit(&h->s, std::move(j));
 }
 
@@ -1303,7 +1318,6 @@ REB_API long reb_amd_server_submit_simulation(struct reb_amd_server* h, struct r
         j->kind = JOB_NBODY;
         j->gravity = r->gravity;
         j->precision = reb_amd_get_precision(r);
-        j->footprint = nbody_footprint(r->N, j->precision, j->gravity);
     } else {
         return fail("only WHFast and leapfrog simulations are served");
     }
@@ -1367,7 +1381,7 @@ REB_API int reb_amd_server_checkpoint(struct reb_amd_server* h, long job, const 
 // Device-memory footprints used for admission.
 REB_API size_t reb_amd_server_whfast_bytes(size_t n_bodies) { return whfast_footprint(n_bodies); }
 REB_API size_t reb_amd_server_nbody_bytes(size_t n, int precision) {
-    return nbody_footprint(n, precision, REB_GRAVITY_BASIC);
+    return nbody_memory(n, precision, REB_GRAVITY_BASIC, SIZE_MAX).bytes;
 }
 
 REB_API int reb_amd_server_status(struct reb_amd_server* h, long job) {
