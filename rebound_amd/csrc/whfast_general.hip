@@ -1163,7 +1163,7 @@ __device__ __forceinline__ void whfast_body(const WHParams& P) {
         }
         synchronize(sys_ok && (P.sync_at_end || (S.req & 1)));
         // the system's flags: any of its lanes' warnings and solver branches
-        for (int o = 1; o < G; o <<= 1) warn |= __shfl_xor(warn, o);
+        warn = group_or(warn, lane - gl, G);
 
         // ---- store
         if (live) {

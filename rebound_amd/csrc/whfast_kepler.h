@@ -29,6 +29,16 @@ static __constant__ double kInvFact[16] = {1.,
                                     1. / 87178291200.,
                                     1. / 1307674368000.};
 
+// The warning bits (0 .. 3) of lanes first .. first + G - 1, a group; groups of any
+// size lie side by side, so exchanges over powers of two would mix neighbours.
+__device__ __forceinline__ int group_or(int warn, int first, int G) {
+    const unsigned long long group = (G < 64 ? (1ull << G) - 1ull : ~0ull) << first;
+    int any = 0;
+    for (int b = 0; b < 4; b++)
+        if (__ballot(warn & (1 << b)) & group) any |= 1 << b;
+    return any;
+}
+
 __device__ __forceinline__ double fastabs(double x) { return (x > 0.) ? x : -x; }
 
 // The number of times z is divided by 4 until |z| <= 0.1

@@ -1042,7 +1042,7 @@ __device__ __forceinline__ void lane_body(const WHParams& P) {
         }
         }
         // the system's flags: any of its lanes' warnings and solver branches
-        for (int o = 1; o < G; o <<= 1) warn |= __shfl_xor(warn, o);
+        warn = group_or(warn, lane - gl, G);
 
         // ---- store
         if (live) {
