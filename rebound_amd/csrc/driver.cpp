@@ -136,16 +136,18 @@ static bool steps_unobserved(const struct reb_simulation* r) {
            r->collision == REB_COLLISION_NONE && !r->N_odes && !r->N_var && r->usleep <= 0;
 }
 
-// A launch holds at most this many steps (about 10 ms), so that an interrupt is
-// seen soon.
-static constexpr size_t kLaunchSteps = 1000;
+// The most WHFast steps that may go into one launch now; 0: step one by one.
+static size_t whfast_most_steps(const struct reb_simulation* r) {
+    if (r->integrator.callbacks.step != rb_whfast_step || !steps_unobserved(r)) return 0;
+    return whfast_launch_steps(r, (const struct reb_integrator_whfast_state*)r->integrator.state);
+}
 
-// Up to n <= kLaunchSteps steps in one launch; one launch per step (metadata
-// copies, two waits, two launches) cost 40 us for an 8-planet system whose step
-// takes 9 us on the device.  Returns the steps done, 0 when the caller has to
-// step one by one.  A refused launch counts as one step, as a refused step does.
+// n steps in one launch; one launch per step (metadata copies, two waits, two
+// launches) cost 40 us for an 8-planet system whose step takes 8 us on the
+// device.  Returns the steps done, 0 when the caller has to step one by one.  A
+// refused launch counts as one step, as a refused step does.
 static size_t whfast_steps_at_once(struct reb_simulation* const r, size_t n) {
-    if (n < 2 || r->integrator.callbacks.step != rb_whfast_step || !steps_unobserved(r)) return 0;
+    if (n < 2) return 0;
     struct timeval t0;
     gettimeofday(&t0, nullptr);
     if (!whfast_steps_device(r, (struct reb_integrator_whfast_state*)r->integrator.state, (long)n)) n = 1;
@@ -307,7 +309,8 @@ REB_API void reb_simulation_steps(struct reb_simulation* const r, size_t N_steps
     begin_call(r);
     run_heartbeat(r);
     for (size_t i = 0; i < N_steps; i++) {
-        const size_t k = whfast_steps_at_once(r, N_steps - i < kLaunchSteps ? N_steps - i : kLaunchSteps);
+        const size_t most = whfast_most_steps(r);
+        const size_t k = whfast_steps_at_once(r, N_steps - i < most ? N_steps - i : most);
         if (k) {
             i += k - 1;
             continue;
@@ -346,7 +349,7 @@ REB_API enum REB_STATUS reb_simulation_integrate(struct reb_simulation* const r,
     if (r->status != REB_STATUS_PAUSED && r->status != REB_STATUS_SCREENSHOT) r->status = REB_STATUS_RUNNING;
     run_heartbeat(r);
     while (reb_check_exit(r, tmax, &last_full_dt) < 0) {
-        const size_t k = whfast_steps_at_once(r, steps_before_exit(r, tmax, kLaunchSteps));
+        const size_t k = whfast_steps_at_once(r, steps_before_exit(r, tmax, whfast_most_steps(r)));
         if (k) {
             if (g_sigint) r->status = REB_STATUS_SIGINT;
             continue;

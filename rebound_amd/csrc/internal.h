@@ -215,6 +215,7 @@ bool check_device_flags(struct reb_simulation* r);           // error words set 
 // WHFast (whfast.hip)
 void whfast_step_device(struct reb_simulation* r, struct reb_integrator_whfast_state* s);
 bool whfast_steps_device(struct reb_simulation* r, struct reb_integrator_whfast_state* s, long n);
+size_t whfast_launch_steps(const struct reb_simulation* r, const struct reb_integrator_whfast_state* s);
 void whfast_synchronize_device(struct reb_simulation* r, struct reb_integrator_whfast_state* s);
 void whfast_release(struct reb_simulation* r);
 void megno_update(struct reb_simulation* r, double dY, double dt_done);   // host_api.cpp

@@ -1,6 +1,8 @@
 """Several WHFast steps in one launch (driver.cpp): the same bodies, time, step
 count and status as stepping one by one, which a heartbeat forces."""
 import ctypes
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -70,4 +72,30 @@ def test_refused_launch_counts_as_steps(gpu):
     with pytest.raises(gpu.RebError):
         sim.steps(5)
     assert sim.s.steps_done == 5 and sim.s.t == 0.0
+    sim.free()
+
+
+def test_stop_is_seen_soon(gpu):
+    """A launch holds about 20 ms of steps: with 64 planets, the lazy kernel and the
+    17th-order corrector in safe mode a step takes 0.12 s, and a launch holds one."""
+    st = np.zeros((65, 11))
+    st[0, 9] = 1.0
+    a, f = 1.0 + 0.2 * np.arange(64), 2.4 * np.arange(64)
+    st[1:, 0], st[1:, 1] = a * np.cos(f), a * np.sin(f)
+    st[1:, 3], st[1:, 4] = -np.sin(f) / np.sqrt(a), np.cos(f) / np.sqrt(a)
+    st[1:, 9] = 1e-9
+    sim = gpu.Sim()
+    sim.set_state(st)
+    w = sim.set_integrator("whfast")
+    w.kernel, w.corrector, w.safe_mode = 3, 17, 1
+    sim.s.dt = 0.05
+    t = threading.Thread(target=lambda: sim.lib.reb_simulation_integrate(sim.ptr, float("inf")))
+    t.start()
+    t0 = time.time()
+    while sim.s.steps_done < 2 and time.time() - t0 < 20:
+        time.sleep(0.001)
+    assert sim.s.steps_done >= 2
+    sim.lib.reb_simulation_stop(sim.ptr)
+    t.join(10)
+    assert not t.is_alive() and sim.s.steps_done < 20
     sim.free()
