@@ -768,6 +768,8 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                 for (int q = 0; q < 4; q++) {
                     const double _r = sqrt(r2[q] + soft2);
                     f[q] = -G / (_r * _r * _r) * c[q].m;
+                    // a filling cell adds nothing, also at distance zero from it
+                    if (k + q >= nr) f[q] = 0.;
                 }
             }
             if ((open[0] | open[1] | open[2] | open[3]) == 0ull) {
