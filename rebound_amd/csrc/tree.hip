@@ -366,7 +366,7 @@ struct __align__(64) GravRec {
     int next, pt;
     double pad;
 };
-// A root box's cell: w2 the width squared, infinite for a leaf (which is always
+// A root box's cell: w2 the width squared, no number for a leaf (which is always
 // walked); its cells are first .. end - 1.
 struct __align__(16) RootRec {
     double x, y, z, m;
@@ -412,7 +412,7 @@ __global__ void k_tree_pack_gravity(const double* __restrict__ nd, const int* __
             if (id >= 0) {
                 const GravRec a = rec(id);
                 rr[nr + __popcll(have & ((1ull << c) - 1ull))] =
-                    RootRec{a.mx, a.my, a.mz, a.m, a.pt < 0 ? a.w * a.w : __builtin_inf(), id, a.next};
+                    RootRec{a.mx, a.my, a.mz, a.m, a.pt < 0 ? a.w * a.w : __builtin_nan(""), id, a.next};
             }
             nr += __popcll(have);
         }
@@ -753,7 +753,9 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                 dy[q] = gy - c[q].y;
                 dz[q] = gz - c[q].z;
                 r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
-                open[q] = __ballot(c[q].w2 > theta2 * r2[q]);
+                // a leaf (no number) always, and a product that is no number, go to the
+                // walk, which leaves out the body's own leaf in every image
+                open[q] = __ballot(!(c[q].w2 <= theta2 * r2[q]));
             }
             unsigned int far = 0;
 #pragma unroll

@@ -97,3 +97,18 @@ def test_gravity_at_the_filling_cells(gpu, orc):
     ref, _ = orc.tree_gravity(st, size, (1, 1, 1), 0.7, 0.0, 1.5, _offsets((size, size), (1, 0)))
     assert np.isfinite(ref).all() and np.array_equal(acc, ref)
     sim.free()
+
+
+@pytest.mark.parametrize("theta2", [0.0, np.inf, np.nan])
+@pytest.mark.parametrize("soft", [0.0, 0.05])
+def test_gravity_angle_limits(gpu, orc, theta2, soft):
+    """Opening angles for which theta^2 r^2 is infinite or no number, with root boxes of
+    one body: the body itself stays left out, in every image."""
+    nr = (6, 5, 1)
+    box = np.array(nr) * 2.0
+    st = _bodies(40, box, 5, 0.2)
+    sim = _sim(gpu, st, 2.0, nr, (1, 1), theta2, soft)
+    acc = sim.update_acceleration()
+    ref, _ = orc.tree_gravity(st, 2.0, nr, 0.7, soft, theta2, _offsets(box, (1, 1)))
+    assert np.isfinite(ref).all() and np.array_equal(acc, ref)
+    sim.free()
