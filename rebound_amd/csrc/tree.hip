@@ -57,6 +57,8 @@ struct GBT {
     double g[kMaxGBT][6];
 };
 
+static constexpr int kRootLds = 256;     // root boxes the collision walk's filter takes (LDS)
+
 struct TreeBuffers {
     size_t last_total = 0;                        // collisions found by the last tree search
     DevBuf key0, key1, idx, key0b, key1b, idxb;   // keys and body permutation
@@ -303,7 +305,7 @@ __global__ void k_tree_nodes(const unsigned long long* __restrict__ k0, const un
         A.next[id] = (e + 1 < n) ? base[e + 1] : total;
         A.pt[id] = -(e - s + 1);
         A.level[id] = d;
-        if (d == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
+        if (roots && d == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
         double cx, cy, cz, w;
         cell_geometry(g, a0, a1, d, cx, cy, cz, w);
         A.cx[id] = cx;
@@ -317,7 +319,7 @@ __global__ void k_tree_nodes(const unsigned long long* __restrict__ k0, const un
     A.next[id] = id + 1;
     A.pt[id] = p;
     A.level[id] = leaf_level;
-    if (leaf_level == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
+    if (roots && leaf_level == 0) roots[(int)(a0 >> (3 * g.L1))] = id;
     double cx, cy, cz, w;
     cell_geometry(g, a0, a1, leaf_level, cx, cy, cz, w);
     A.cx[id] = cx;
@@ -366,8 +368,8 @@ struct __align__(64) GravRec {
     int next, pt;
     double pad;
 };
-// A root box's cell: w2 the width squared, no number for a leaf (which is always
-// walked); its cells are first .. end - 1.
+// A root box's cell: w2 the width squared; its cells are first .. end - 1.  A leaf
+// (a single cell): w2 no number, end its body's complement.
 struct __align__(16) RootRec {
     double x, y, z, m;
     double w2;
@@ -384,13 +386,19 @@ struct __align__(64) CollCell {
     double v[3];
 };
 
-// The walk records of all cells.  The first wavefront also writes the root
+// The walk records of all cells.  The first workgroup also writes the root
 // boxes' cells, empty boxes left out, their number, and up to three massless
 // cells far away behind them (accepted by every body, without effect), so that
-// the walk can read them in fours.
-__global__ void k_tree_pack_gravity(const double* __restrict__ nd, const int* __restrict__ ni, size_t cap, int total,
-                                    GravRec* __restrict__ g, const int* __restrict__ roots, int nroot,
-                                    RootRec* __restrict__ rr, int* __restrict__ nroots) {
+// the walk can read them in fours.  It finds them in the list of the root boxes
+// or, if that would be longer (roots null: a grid of mostly empty boxes), among the
+// bodies in key order, of which the first of a root box shares no digit with
+// the one before it; 1024 entries at a time.
+__global__ __launch_bounds__(256) void k_tree_pack_gravity(const double* __restrict__ nd, const int* __restrict__ ni,
+                                                           size_t cap, int total, GravRec* __restrict__ g,
+                                                           const int* __restrict__ roots, int nroot,
+                                                           const int* __restrict__ lcp, const int* __restrict__ base,
+                                                           int n, RootRec* __restrict__ rr,
+                                                           int* __restrict__ nroots) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     auto rec = [&](int k) {
         GravRec a;
@@ -404,17 +412,41 @@ __global__ void k_tree_pack_gravity(const double* __restrict__ nd, const int* __
         a.pad = 0.;
         return a;
     };
-    if (c < 64) {
+    if (blockIdx.x == 0) {
+        __shared__ int found[4];
+        const int w = c >> 6, lane = c & 63;
+        const int entries = roots ? nroot : n;
         int nr = 0;
-        for (int q = 0; q < nroot; q += 64) {
-            const int id = q + c < nroot ? roots[q + c] : -1;
-            const unsigned long long have = __ballot(id >= 0);
-            if (id >= 0) {
-                const GravRec a = rec(id);
-                rr[nr + __popcll(have & ((1ull << c) - 1ull))] =
-                    RootRec{a.mx, a.my, a.mz, a.m, a.pt < 0 ? a.w * a.w : __builtin_nan(""), id, a.next};
+        for (int q0 = 0; q0 < entries; q0 += 1024) {
+            int id[4], mine = 0;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int q = q0 + 4 * c + u;
+                id[u] = -1;
+                if (q < entries) id[u] = roots ? roots[q] : (q == 0 || lcp[q - 1] < 0 ? base[q] : -1);
+                mine += id[u] >= 0;
             }
-            nr += __popcll(have);
+            int upto = mine;                         // in the wavefront, this lane included
+            for (int off = 1; off < 64; off <<= 1) {
+                const int v = __shfl_up(upto, off);
+                if (lane >= off) upto += v;
+            }
+            if (lane == 63) found[w] = upto;
+            __syncthreads();
+            int at = nr + upto - mine;
+            for (int v = 0; v < 4; v++) {
+                if (v < w) at += found[v];
+                nr += found[v];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if (id[u] < 0) continue;
+                const GravRec a = rec(id[u]);
+                const bool leaf = a.pt >= 0;
+                rr[at++] = RootRec{a.mx, a.my, a.mz, a.m, leaf ? __builtin_nan("") : a.w * a.w, id[u],
+                                   leaf ? ~a.pt : a.next};
+            }
+            __syncthreads();
         }
         if (c < 3) rr[nr + c] = RootRec{0x1p66, 0., 0., 0., 0., 0, 0};
         if (c == 0) *nroots = nr;
@@ -537,7 +569,10 @@ bool tree_build(struct reb_simulation* r, TreeFor what) {
     const int n = (int)r->N;
     if (!tree_alloc(r, T, n ? n : 1)) return false;
     TreeGeom g = tree_geom(r, T);
-    if (!T->roots.ensure(sizeof(int) * (size_t)T->nroot)) {
+    // The root boxes' cells are listed by box unless most boxes are empty (the
+    // collision search reads the list of up to kRootLds boxes).
+    const bool by_box = T->nroot <= std::max(n, kRootLds);
+    if (by_box && !T->roots.ensure(sizeof(int) * (size_t)T->nroot)) {
         reb_simulation_error(r, "Out of device memory for the tree.");
         return false;
     }
@@ -551,7 +586,8 @@ bool tree_build(struct reb_simulation* r, TreeFor what) {
         if (n == 0) break;
         hipLaunchKernelGGL(k_tree_keys, dim3((n + 255) / 256), dim3(256), 0, d->stream, d->field(FX), d->field(FY),
                            d->field(FZ), n, g, two ? 1 : 0, T->key0.as<unsigned long long>(),
-                           T->key1.as<unsigned long long>(), T->idx.as<int>(), info, T->roots.as<int>(), T->nroot);
+                           T->key1.as<unsigned long long>(), T->idx.as<int>(), info, T->roots.as<int>(),
+                           by_box ? T->nroot : 0);
         if (!tree_sort(r, T, n, two)) return false;
         hipLaunchKernelGGL(k_tree_lcp, dim3((n + 255) / 256), dim3(256), 0, d->stream,
                            T->key0.as<unsigned long long>(), T->key1.as<unsigned long long>(), n, g.L1, g.L2,
@@ -608,10 +644,10 @@ bool tree_build(struct reb_simulation* r, TreeFor what) {
                        T->key0.as<unsigned long long>(), T->key1.as<unsigned long long>(), T->idx.as<int>(),
                        T->lcp.as<int>(), T->base.as<int>(), n, total, g, two ? 1 : 0, T->node_d.as<double>(),
                        T->node_i.as<int>(), T->node_cap, d->field(FM), d->field(FX), d->field(FY), d->field(FZ),
-                       T->roots.as<int>());
+                       by_box ? T->roots.as<int>() : nullptr);
     const dim3 cells((total + 255) / 256);
     if (!(what == TREE_GRAVITY ? T->grec.ensure(sizeof(GravRec) * (size_t)total) &&
-                                     T->root_rec.ensure(sizeof(RootRec) * ((size_t)T->nroot + 3))
+                                     T->root_rec.ensure(sizeof(RootRec) * ((size_t)std::min(T->nroot, n) + 3))
                                : T->crec.ensure(sizeof(CollCell) * (size_t)total))) {
         reb_simulation_error(r, "Out of device memory for the tree cells.");
         return false;
@@ -621,8 +657,9 @@ bool tree_build(struct reb_simulation* r, TreeFor what) {
             hipLaunchKernelGGL(k_tree_moments, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
                                T->node_i.as<int>(), T->node_cap, total, lev);
         hipLaunchKernelGGL(k_tree_pack_gravity, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
-                           T->node_i.as<int>(), T->node_cap, total, T->grec.as<GravRec>(), T->roots.as<int>(),
-                           T->nroot, T->root_rec.as<RootRec>(), info + 3);
+                           T->node_i.as<int>(), T->node_cap, total, T->grec.as<GravRec>(),
+                           by_box ? T->roots.as<int>() : nullptr, T->nroot, T->lcp.as<int>(), T->base.as<int>(), n,
+                           T->root_rec.as<RootRec>(), info + 3);
     } else {
         hipLaunchKernelGGL(k_tree_pack_collide, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
                            T->node_i.as<int>(), T->node_cap, total, T->crec.as<CollCell>(), d->field(FX), d->field(FY),
@@ -753,8 +790,7 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                 dy[q] = gy - c[q].y;
                 dz[q] = gz - c[q].z;
                 r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
-                // a leaf (no number) always, and a product that is no number, go to the
-                // walk, which leaves out the body's own leaf in every image
+                // leaves, and products that are no number, count as opened
                 open[q] = __ballot(!(c[q].w2 <= theta2 * r2[q]));
             }
             unsigned int far = 0;
@@ -787,9 +823,12 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if (k + q >= nr) break;
-                if (open[q]) {
+                if (open[q] && c[q].end >= 0) {
                     walk(c[q].first, c[q].end, gx, gy, gz);
-                } else {
+                } else if (me != ~c[q].end) {
+                    // a cell that no body opens, or a leaf, which its own body leaves
+                    // out in every image (a cell's end is positive, its complement
+                    // no body)
                     a_x += f[q] * dx[q];
                     a_y += f[q] * dy[q];
                     a_z += f[q] * dz[q];
@@ -952,8 +991,6 @@ struct RootBox {
     double x, y, z, w;
     int first, end, leaf, pad;
 };
-
-static constexpr int kRootLds = 256;     // root boxes the filter takes (LDS)
 
 // Records kept per body by the single-pass search; the bodies with more
 // collisions are searched again by a pass that walks only them.

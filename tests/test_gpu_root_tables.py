@@ -112,3 +112,43 @@ def test_gravity_angle_limits(gpu, orc, theta2, soft):
     ref, _ = orc.tree_gravity(st, 2.0, nr, 0.7, soft, theta2, _offsets(box, (1, 1)))
     assert np.isfinite(ref).all() and np.array_equal(acc, ref)
     sim.free()
+
+
+@pytest.mark.parametrize("nr,n", [((32, 32, 1), 1500), ((33, 31, 1), 12000), ((128, 128, 1), 900),
+                                  ((129, 128, 1), 900), ((1000, 1000, 1), 300), ((1, 20000, 1), 2)])
+def test_large_root_grids(gpu, orc, nr, n):
+    """Root grids of one and more batches of the compaction (1024 boxes), listed by box
+    and (more boxes than bodies) by body; the device memory of a tree does not grow with
+    empty boxes."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so", mode=ctypes.RTLD_GLOBAL)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_memory():
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    box = np.array(nr) * 2.0
+    st = _bodies(n, box, n)
+    st[:, 10] *= 0.3
+    sim = _sim(gpu, st, 2.0, nr, (1, 0), 0.4, 0.05)
+    before = free_memory()
+    acc = sim.update_acceleration()
+    assert before - free_memory() <= (64 << 20)
+    ref, _ = orc.tree_gravity(st, 2.0, nr, 0.7, 0.05, 0.4, _offsets(box, (1, 0)))
+    assert np.array_equal(acc, ref)
+    s = sim.s
+    s.gravity = gpu.GRAVITY["none"]
+    s.collision = gpu.COLLISION["tree"]
+    found = []
+    from rebound_amd import _abi
+    keep = _abi.RESOLVE(lambda r, c: found.append((c.p1, c.p2)) or 0)
+    s.collision_resolve = keep
+    sim.set_integrator("leapfrog")
+    s.dt = 0.0
+    sim.steps(1)
+    gb6 = np.hstack([_offsets(box, (1, 0)), np.zeros((3, 3))])
+    ref = orc.collisions_tree(st, 2.0, nr, gb6)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    assert sorted(found) == sorted((int(a), int(b)) for a, b in np.asarray(ref)[:, :2])
+    sim.free()
