@@ -392,12 +392,13 @@ struct __align__(64) CollCell {
 // the walk can read them in fours.  It finds them in the list of the root boxes
 // or, if that would be longer (roots null: a grid of mostly empty boxes), among the
 // bodies in key order, of which the first of a root box shares no digit with
-// the one before it; 1024 entries at a time.
+// the one before it; 1024 entries at a time.  Without a table (walk_table) all cells
+// are one record, which every body opens.
 __global__ __launch_bounds__(256) void k_tree_pack_gravity(const double* __restrict__ nd, const int* __restrict__ ni,
                                                            size_t cap, int total, GravRec* __restrict__ g,
                                                            const int* __restrict__ roots, int nroot,
                                                            const int* __restrict__ lcp, const int* __restrict__ base,
-                                                           int n, RootRec* __restrict__ rr,
+                                                           int n, int table, RootRec* __restrict__ rr,
                                                            int* __restrict__ nroots) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     auto rec = [&](int k) {
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(256) void k_tree_pack_gravity(const double* __restr
     if (blockIdx.x == 0) {
         __shared__ int found[4];
         const int w = c >> 6, lane = c & 63;
-        const int entries = roots ? nroot : n;
+        const int entries = !table ? 0 : (roots ? nroot : n);
         int nr = 0;
         for (int q0 = 0; q0 < entries; q0 += 1024) {
             int id[4], mine = 0;
@@ -447,6 +448,10 @@ __global__ __launch_bounds__(256) void k_tree_pack_gravity(const double* __restr
                                    leaf ? ~a.pt : a.next};
             }
             __syncthreads();
+        }
+        if (!table) {
+            if (c == 0) rr[0] = RootRec{0., 0., 0., 0., __builtin_nan(""), 0, total};
+            nr = 1;
         }
         if (c < 3) rr[nr + c] = RootRec{0x1p66, 0., 0., 0., 0., 0, 0};
         if (c == 0) *nroots = nr;
@@ -558,7 +563,7 @@ static bool tree_sort(struct reb_simulation* r, TreeBuffers* T, int n, bool two)
 // search with its own records (its tests read no moments, which take a launch per
 // level).
 enum TreeFor { TREE_GRAVITY, TREE_COLLISIONS };
-bool tree_build(struct reb_simulation* r, TreeFor what) {
+bool tree_build(struct reb_simulation* r, TreeFor what, bool table = true) {
     DeviceState* d = dev_of(r);
     if (r->root_size <= 0.0) {
         reb_simulation_error(r, "Set root_size to a finite value to use a tree based gravity or collision solver.");
@@ -659,7 +664,7 @@ bool tree_build(struct reb_simulation* r, TreeFor what) {
         hipLaunchKernelGGL(k_tree_pack_gravity, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
                            T->node_i.as<int>(), T->node_cap, total, T->grec.as<GravRec>(),
                            by_box ? T->roots.as<int>() : nullptr, T->nroot, T->lcp.as<int>(), T->base.as<int>(), n,
-                           T->root_rec.as<RootRec>(), info + 3);
+                           table ? 1 : 0, T->root_rec.as<RootRec>(), info + 3);
     } else {
         hipLaunchKernelGGL(k_tree_pack_collide, cells, dim3(256), 0, d->stream, T->node_d.as<double>(),
                            T->node_i.as<int>(), T->node_cap, total, T->crec.as<CollCell>(), d->field(FX), d->field(FY),
@@ -691,30 +696,44 @@ static int walk_bodies(int n) {
     return w;
 }
 
+// Whether the gravity walk goes by the table of root boxes: with fewer records than
+// this (boxes times images) most of a body's terms come from opened boxes, whose
+// cells one walk in block order reads without a restart per box (64 boxes, 50000
+// bodies: 777 us a step by the table, 677 by one walk; 100 boxes, 200000: 1212, 1110;
+// 4 boxes x 25 images, 100000: 1233, 1183).  Above it the table wins (196 boxes, 20000:
+// 418, 441; 9 boxes x 25 images, 12007: 638, 646; 36 x 25, 12007: 643, 777).
+static constexpr double kTableRecords = 150;
+static bool walk_table(const struct reb_simulation* r, size_t images) {
+    const double boxes = std::min((double)r->N_root_x * r->N_root_y * r->N_root_z, (double)r->N);
+    return boxes * images >= kTableRecords;
+}
+
 // tree.c:275-328 for every ghost box (gravity.c:84-102), in the reference's
 // expressions; `width` bodies (in key order) per wavefront.
 //
-// Most of a body's terms are whole root boxes (200000 bodies in 100 root boxes
-// with 25 images: 2500 of 2855).  The wavefront reads their records four at a
-// time from a table (uniform, in the scalar cache).  Four that no lane opens are
-// evaluated together, four independent square root and division chains, and added in
-// order; a root box that some lane opens is walked along the pre-order, cell by
-// cell.  The square roots and divisions are the short sequences of
-// ieee_mid.h, or the compiler's if an operand is out of their range.  200000
-// bodies: 2.43 ms one cell at a time, now 1.9; what bounds it is the latency of the
-// near part's cell fetches and the FP64 issue of the wavefronts of the SIMDs that hold
-// four (3125 wavefronts on 1024 SIMDs).
+// With many root boxes or images most of a body's terms are whole root boxes
+// (200000 bodies in 100 root boxes with 25 images: 2500 of 2855).  The wavefront
+// reads their records four at a time from a table (uniform, in the scalar
+// cache).  Four that no lane opens are evaluated together, four independent chains
+// of the short square root and division of ieee_mid.h (or the compiler's if an
+// operand is out of their range), and added in order.  A root box that some lane
+// opens is walked along the pre-order, cell by cell, with the compiler's sequences:
+// the choice between the two cost a walk 10 %.  What bounds it is the latency of
+// the near part's cell fetches and the FP64 issue of the wavefronts of the SIMDs that
+// hold four (200000 bodies: 3125 wavefronts on 1024 SIMDs).  Ring patches of 12007 and
+// 100000 bodies in 36 root boxes, a step without collisions: 896 and 1490 us one cell at a
+// time, now 643 and 1279.  xcd: the bodies of one XCD are neighbours (with the table).
 __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__ rec, int total,
                                                      const RootRec* __restrict__ root,
                                                      const int* __restrict__ nroots, const int* __restrict__ idx,
-                                                     int n, int width, const double* __restrict__ x,
+                                                     int n, int width, int xcd, const double* __restrict__ x,
                                                      const double* __restrict__ y, const double* __restrict__ z,
                                                      GBT gl, double G, double soft2, double theta2,
                                                      double* __restrict__ ax, double* __restrict__ ay,
                                                      double* __restrict__ az,
                                                      unsigned long long* __restrict__ counter) {
     const int lane = threadIdx.x;
-    const int s = xcd_block() * width + lane;
+    const int s = (xcd ? xcd_block() : (int)blockIdx.x) * width + lane;
     if (s - lane >= n) return;                       // one wave per block: uniform
     const bool live = lane < width && s < n;
     const int me = live ? idx[s] : -1;
@@ -755,16 +774,8 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                     use = false;
                 }
                 if (use) {
-                    const double rs = r2 + soft2;
-                    double f;
-                    if (g_mid && mid_distance(rs) < kMidSpan) {
-                        const double _r = sqrt_mid(rs);
-                        f = div_mid(-G, _r * _r * _r);
-                    } else {
-                        const double _r = sqrt(rs);
-                        f = -G / (_r * _r * _r);
-                    }
-                    const double prefact = f * cur.m;
+                    const double _r = sqrt(r2 + soft2);
+                    const double prefact = -G / (_r * _r * _r) * cur.m;
                     a_x += prefact * dx;
                     a_y += prefact * dy;
                     a_z += prefact * dz;
@@ -780,7 +791,7 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
         const double gx = gl.g[g][0] + xi, gy = gl.g[g][1] + yi, gz = gl.g[g][2] + zi;
         for (int k = 0; k < nr; k += 4) {
             RootRec c[4];
-            double dx[4], dy[4], dz[4], r2[4], f[4];
+            double dx[4], dy[4], dz[4], r2[4];
             unsigned long long open[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) c[q] = root[k + q];
@@ -793,24 +804,25 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                 // leaves, and products that are no number, count as opened
                 open[q] = __ballot(!(c[q].w2 <= theta2 * r2[q]));
             }
-            unsigned int far = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const double rs = r2[q] + soft2;
-                far = max(far, mid_distance(rs));
-                const double _r = sqrt_mid(rs);
-                f[q] = div_mid(-G, _r * _r * _r) * c[q].m;
-            }
-            if (!g_mid || __any(far >= kMidSpan)) {
+            if ((open[0] | open[1] | open[2] | open[3]) == 0ull) {
+                unsigned int far = 0;
+                double f[4];
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const double _r = sqrt(r2[q] + soft2);
-                    f[q] = -G / (_r * _r * _r) * c[q].m;
-                    // a filling cell adds nothing, also at distance zero from it
-                    if (k + q >= nr) f[q] = 0.;
+                    const double rs = r2[q] + soft2;
+                    far = max(far, mid_distance(rs));
+                    const double _r = sqrt_mid(rs);
+                    f[q] = div_mid(-G, _r * _r * _r) * c[q].m;
                 }
-            }
-            if ((open[0] | open[1] | open[2] | open[3]) == 0ull) {
+                if (!g_mid || __any(far >= kMidSpan)) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const double _r = sqrt(r2[q] + soft2);
+                        f[q] = -G / (_r * _r * _r) * c[q].m;
+                        // a filling cell adds nothing, also at distance zero from it
+                        if (k + q >= nr) f[q] = 0.;
+                    }
+                }
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     a_x += f[q] * dx[q];
@@ -829,9 +841,11 @@ __global__ __launch_bounds__(64) void k_tree_gravity(const GravRec* __restrict__
                     // a cell that no body opens, or a leaf, which its own body leaves
                     // out in every image (a cell's end is positive, its complement
                     // no body)
-                    a_x += f[q] * dx[q];
-                    a_y += f[q] * dy[q];
-                    a_z += f[q] * dz[q];
+                    const double _r = sqrt(r2[q] + soft2);
+                    const double prefact = -G / (_r * _r * _r) * c[q].m;
+                    a_x += prefact * dx[q];
+                    a_y += prefact * dy[q];
+                    a_z += prefact * dz[q];
                     inter++;
                 }
             }
@@ -854,11 +868,12 @@ bool gravity_tree(struct reb_simulation* r) {
     DeviceState* d = dev_of(r);
     // gravity.c:54-56: wrap into the box before building
     if (!boundary_device(r)) return false;
-    if (!tree_build(r, TREE_GRAVITY)) return false;
+    auto gbv = ghostboxes(r, r->N_ghost_x, r->N_ghost_y, r->N_ghost_z);
+    const bool table = walk_table(r, gbv.size());
+    if (!tree_build(r, TREE_GRAVITY, table)) return false;
     TreeBuffers* T = d->tree;
     const int n = (int)r->N;
     if (n == 0) return true;
-    auto gbv = ghostboxes(r, r->N_ghost_x, r->N_ghost_y, r->N_ghost_z);
     if ((int)gbv.size() > kMaxGBT) {
         reb_simulation_error(r, "Too many ghost boxes for tree gravity (at most 64).");
         return false;
@@ -878,7 +893,8 @@ bool gravity_tree(struct reb_simulation* r) {
     const int width = walk_bodies(n);
     const dim3 grid = xcd_grid((n + width - 1) / width);
     hipLaunchKernelGGL(k_tree_gravity, grid, dim3(64), 0, d->stream, T->grec.as<GravRec>(), T->nnodes,
-                       T->root_rec.as<RootRec>(), T->info.as<int>() + 3, T->idx.as<int>(), n, width, d->field(FX), d->field(FY), d->field(FZ), gl, r->G,
+                       T->root_rec.as<RootRec>(), T->info.as<int>() + 3, T->idx.as<int>(), n, width, table ? 1 : 0, d->field(FX),
+                       d->field(FY), d->field(FZ), gl, r->G,
                        r->softening * r->softening, r->opening_angle2, d->field(FAX), d->field(FAY), d->field(FAZ),
                        counter);
     mark_device_newer(r);

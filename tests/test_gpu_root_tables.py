@@ -89,12 +89,12 @@ def test_collisions(gpu, orc, nr, n, cluster, negative):
 def test_gravity_at_the_filling_cells(gpu, orc):
     """The records that fill the table to fours lie at (2^66, 0, 0): the image of a
     body at the origin of a box of that size is exactly there, without softening."""
-    size = 2.0 ** 66
-    st = _bodies(40, np.full(3, 2.0 ** 55), 3)
+    size, nr = 2.0 ** 60, (64, 1, 1)
+    st = _bodies(200, np.full(3, 2.0 ** 55), 3)
     st[7, :3] = 0.0
-    sim = _sim(gpu, st, size, (1, 1, 1), (1, 0), 1.5, 0.0)
+    sim = _sim(gpu, st, size, nr, (1, 0), 1.5, 0.0)
     acc = sim.update_acceleration()
-    ref, _ = orc.tree_gravity(st, size, (1, 1, 1), 0.7, 0.0, 1.5, _offsets((size, size), (1, 0)))
+    ref, _ = orc.tree_gravity(st, size, nr, 0.7, 0.0, 1.5, _offsets((64 * size, size), (1, 0)))
     assert np.isfinite(ref).all() and np.array_equal(acc, ref)
     sim.free()
 
