@@ -1691,8 +1691,11 @@ __global__ __launch_bounds__(64) void k_energy_fold_terms(const double* __restri
 // lanes' sums are added with their rounding errors kept (two_add).  Tiles are
 // spread over blockIdx.y: with one workgroup per 256 targets walking its whole
 // triangle row the first one set the time (65536 bodies 12.5 ms, 10007 1.94, 1024 0.216;
-// now 1.80, 0.084 and 0.047, the call's copy and wait included).  A lane whose sum is NaN (coincident, non-finite or
-// overflowing distances) repeats its tile with IEEE arithmetic.
+// now 1.80, 0.084 and 0.047, the call's copy and wait included).  A lane whose sum is not
+// finite (coincident, non-finite or overflowing distances, or squares of distances below
+// the normal range, whose reciprocal overflows in the refinement) repeats its tile with
+// IEEE arithmetic.
+
 // Sum of (s, c) over the workgroup's threads into out[0] (sum) and out[1] (its
 // rounding error), in a fixed order.
 template <int THREADS>
@@ -1755,7 +1758,7 @@ __global__ __launch_bounds__(256) void k_energy_tiles(const double* __restrict__
             c = (tv - s) - yv;
             s = tv;
         }
-        if (s != s) {
+        if (!(fabs(s) < __builtin_inf())) {
             s = s0;
             c = c0s;
             for (int k = first; k < n; k++) {

@@ -75,3 +75,19 @@ def test_overflow_and_coincidence(gpu):
     sim = _sim(gpu, st)
     assert not np.isfinite(sim.energy())
     sim.free()
+
+
+@pytest.mark.parametrize("n,i,j", [(2, 0, 1), (256, 254, 255), (257, 0, 256), (600, 3, 511), (600, 100, 101)])
+def test_distance_below_the_normal_range(gpu, n, i, j):
+    """A pair whose squared distance is subnormal, also as the last source of a tile:
+    finite, with the value of FP64 arithmetic (the square keeps few bits, so the
+    reference forms it the same way)."""
+    st = _bodies(n, n)
+    st[i, :3] = 0.0
+    st[j, :3] = [1e-160, 0.0, 0.0]
+    st[[i, j], 9] = 1e-78                          # the pair's term: about 1e4
+    kin, pot = _long(np.delete(st, [i, j], 0), n - 2, n - 2)
+    near = 1e-78 * 1e-78 / np.sqrt(1e-160 * 1e-160)
+    sim = _sim(gpu, st)
+    assert abs(sim.energy() - float(kin + pot) + near) <= 8 * 2.0 ** -53 * max(kin, -pot, near)
+    sim.free()
