@@ -1799,9 +1799,14 @@ __global__ __launch_bounds__(1024) void k_energy_total(const double* __restrict_
 }
 
 // Source tiles of a target tile spread over this many workgroups: one tile each
-// up to 128 tiles, and the partial sums (two doubles each, and two per target
-// tile) fit the 2 n + 16 doubles of the caller's scratch.
-static int energy_split(int tiles) { return tiles < 128 ? tiles : 128 - 1; }
+// up to 127 tiles, and the partial sums (two doubles each, and two per target
+// tile, after the first 16) fit the caller's scratch.
+static constexpr int energy_split(int tiles) { return tiles < 128 ? tiles : 128 - 1; }
+static constexpr bool energy_fits(int tiles) {      // the fewest bodies of so many tiles
+    return 16 + 2 * (size_t)tiles * (energy_split(tiles) + 1) <= energy_scratch(256 * (size_t)(tiles - 1) + 1);
+}
+static constexpr bool energy_fits_upto(int tiles) { return tiles < 1 || (energy_fits(tiles) && energy_fits_upto(tiles - 1)); }
+static_assert(energy_fits_upto(400) && energy_fits(4096) && energy_fits(1 << 20), "energy scratch");
 
 int energy_launch(const double* x, const double* y, const double* z, const double* vx, const double* vy,
                   const double* vz, const double* m, int n, int n_active, int n_interact, double G, bool exact,
@@ -1858,7 +1863,7 @@ double energy_device(struct reb_simulation* r) {
                                "can differ from the reference's.");
     }
     const size_t terms_cap = exact ? std::min<size_t>(kEnergyTermsMax, N_active * N_interact / 2 + N_interact) : 0;
-    const size_t head = 2 * N + 16;
+    const size_t head = energy_scratch(N);
     if (!d->scratch.ensure(sizeof(double) * (head + terms_cap))) {
         reb_simulation_error(r, "Out of device memory for the energy reduction.");
         return nan("");

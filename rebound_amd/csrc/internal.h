@@ -194,7 +194,8 @@ int seg_step_launch(const SegJob* jobs, const SegRange* ranges, int nranges, con
                     hipStream_t st);
 int seg_fast_mode(int precision, int compensated);
 // Energy (tools.c:108-162) of device arrays into out[0] (kinetic) and out[1]
-// (potential) on the stream; `scratch` holds 2 n + 16 doubles.
+// (potential) on the stream; `out` holds energy_scratch(n) doubles.
+constexpr size_t energy_scratch(size_t n) { return 2 * n + 18; }
 int energy_launch(const double* x, const double* y, const double* z, const double* vx, const double* vy,
                   const double* vz, const double* m, int n, int n_active, int n_interact, double G, bool exact,
                   double* scratch, hipStream_t st, double* terms = nullptr, size_t terms_cap = 0);

@@ -860,7 +860,7 @@ static bool nb_admit(Server* S, Job* j) {
     size_t ws = 0;
     seg_plan((int)n, &j->chunk, &j->used, &ws);
     if (!j->soa.ensure(sizeof(double) * 10 * n) || !j->partial.ensure(ws) ||
-        !j->scratch.ensure(sizeof(double) * (2 * n + 16)))
+        !j->scratch.ensure(sizeof(double) * energy_scratch(n)))
         return nb_fail(S, "out of device memory");
     if (!S->nb_meta.ensure(sizeof(double) * 10 * n + 64)) return nb_fail(S, "staging");
     double* h = static_cast<double*>(S->nb_meta.p);
