@@ -1275,15 +1275,24 @@ static int max_chunks(int n_recv, int n_src, int ngb) {
     return s;
 }
 // max_chunks rounds up, so that at many sizes a few workgroups more than the 2048
-// of two full rounds (four wavefronts on every SIMD) start a third: one chunk
-// fewer then (30011 targets, 20011 sources, FP64: 489 us with 118 x 18 workgroups, 469
-// with 118 x 17).  With half a workgroup per CU or more left over the third round
-// is worth its chunks (65000 targets, 20000 sources: 930 us with 254 x 9, 942 with 254
-// x 8).
+// of two full rounds (four wavefronts on every SIMD) start a third: the last chunk's.
+// One chunk fewer then, if that chunk is nearly a full one (a short one costs
+// little) and the others do not grow by more than the third round takes, about an
+// eighth.  Measured, us with and without the chunk, targets / sources, FP64: last
+// chunk 0.71 to 1 of the others, which grow by 4 to 10 %: 27548 / 27548 520 and 499,
+// 30011 / 20011 489 and 469, 34972 844 and 796, 40348 1108 and 1060, 47772 1512 and 1496;
+// growth 12 %: 58268 2241 and 2268; last chunk 0.1 to 0.65: 13468 147 and 154, 18332 /
+// 9166 133 and 143, 21660 / 10830 177 and 187; chunks below 700 sources, whose lengths
+// round up by more: 25105 / 6705 132 and 140, 16628 / 16245 195 and 208.  With half a workgroup per CU or more left
+// over the third round is worth its chunks (65000 / 20000: 930 with 254 x 9, 942 with
+// 254 x 8).
 static int pick_chunks(int n_recv, int n_src, int ngb) {
     const int s = max_chunks(n_recv, n_src, ngb);
     const long blocks = (n_recv + kFast - 1) / kFast;
-    return s > 2 && blocks * s > 2048 && blocks * s <= 2048 + 128 ? s - 1 : s;
+    if (s <= 2 || blocks * s <= 2048 || blocks * s > 2048 + 128) return s;
+    const int c = round_chunk((n_src + s - 1) / s), longer = round_chunk((n_src + s - 2) / (s - 1));
+    const int last = n_src - (s - 1) * c;              // none left if rounding made the chunks longer
+    return c >= 700 && 10L * last >= 7L * c && 100L * longer <= 112L * c ? s - 1 : s;
 }
 
 static size_t workspace_bytes(int n, int nchunk) { return sizeof(double) * 6 * (size_t)n * (size_t)nchunk; }
