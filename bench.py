@@ -101,7 +101,9 @@ def run_mode(amd, args, name, precision, gravity, steps, warmup):
     kernel_ms = ktot.value / max(kn.value, 1)
     # ordered pairs the timed kernel evaluates per launch: N(N-1) for the
     # one-sided kernels; for the pair-symmetric one the pairs between
-    # superblocks, each unordered pair once (counted here as two ordered)
+    # superblocks, each unordered pair once (counted here as two ordered); its
+    # launch also evaluates the pairs inside superblocks (1.6 % at N=65536), which
+    # are not counted, so its rate and roofline are understated by as much
     kp = kpairs / max(kn.value, 1)
     sym = kp < pairs
     if sym:
